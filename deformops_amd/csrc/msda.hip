@@ -829,6 +829,20 @@ struct BwdGeom {
                     // every kernel decides the same way with chunked_sort()
 };
 
+// The sample records of the one-launch sort (msda_record_sort_kernel), in bucket order
+// per chunk of queries: three streams (location pairs, weights, query numbers inside
+// the chunk) and each chunk's bucket offsets. Sample region of (b, h) and chunk c:
+// (b H + h) Q L P + c qc L P, at most qc L P records.
+struct Records {
+  char* loc;       // location pairs, in the location dtype
+  char* w;         // attention weights: RecordWeight
+  uint16_t* q;     // query - c qc
+  uint16_t* offs;  // per (b, h, chunk): the first record of every bucket, then the end
+  int* queue;      // the matrix-core kernel's kXcds work-queue counters, one per 128-byte line
+  int64_t offs_cap;  // entries the offsets' memory holds
+  int qc, nch;     // queries per chunk, chunks per (b, h)
+};
+
 struct LevelTiles {
   int lh, lw;     // log2 of the tile height and width
   int ntx, nty;   // tiles across and down
@@ -847,48 +861,53 @@ __device__ inline int log2_ceil(int v) {
   return r;
 }
 
-// Tiles of every level (one thread). Tile sides are powers of two, so that tiles
-// and sub-buckets follow from shifts and masks; a tile may reach past the level's
-// right or bottom edge. Returns the tile count of one (b, h), or -1 when it exceeds
-// 2^29.
-__device__ inline int64_t plan_tiles(const Problem& p, const BwdGeom& bg, const Level* levels,
-                                     LevelTiles* lt) {
-  int64_t total = 0;
-  const int64_t records = 4 * int64_t(p.Q) * p.P;
-  for (int l = 0; l < p.L; ++l) {
-    const Level lv = levels[l];
-    LevelTiles t{0, 0, 0, 0, int(total)};
-    if (lv.ok && bg.sub_log2 > 0) {
-      int side = bg.sub_log2;
-      // A level with few tasks of many candidates (a coarse level of a small call)
-      // takes 4 x 4 tiles, one MFMA sub-tile each: four times the tasks, each with
-      // about a third of the candidates, so that they do not run long after the other
-      // levels' tasks (the call waits for its longest task).
-      if (bg.small_tiles) {
-        const int64_t t8 = int64_t((lv.w + 7) >> 3) * ((lv.h + 7) >> 3);
-        const int64_t kblocks = int64_t(p.Q) * p.P * 13 / (10 * 64 * t8);  // per 8 x 8 task, expected
-        if (int64_t(p.B) * p.H * t8 < kSmallTileTasks && kblocks >= kSmallTileKBlocks) side = 2;
-      }
-      t.lw = t.lh = side;
-      t.ntx = (lv.w + (1 << t.lw) - 1) >> t.lw;
-      t.nty = (lv.h + (1 << t.lh) - 1) >> t.lh;
-    } else if (lv.ok) {
-      const int64_t hw = int64_t(lv.h) * lv.w;
-      const int64_t want = records > 0 ? int64_t(kTargetRecords) * hw / records : bg.cap;
-      const int a = pow2_floor(std::min<int64_t>(std::max<int64_t>(want, bg.amin), bg.cap));
-      int tw0 = 1;
-      while (tw0 * tw0 < a) tw0 *= 2;
-      const int wcap = 1 << log2_ceil(lv.w), hcap = 1 << log2_ceil(lv.h);
-      int tw = min(wcap, tw0);
-      const int th = min(hcap, max(1, a / tw));
-      tw = min(wcap, max(tw, a / th));
-      t.lw = log2_ceil(tw);
-      t.lh = log2_ceil(th);
-      t.ntx = (lv.w + tw - 1) >> t.lw;
-      t.nty = (lv.h + th - 1) >> t.lh;
+// Tiles of one level. Tile sides are powers of two, so that tiles and sub-buckets
+// follow from shifts and masks; a tile may reach past the level's right or bottom
+// edge. `base` is left to number_tiles.
+__device__ inline LevelTiles level_tiles(const Problem& p, const BwdGeom& bg, const Level& lv) {
+  LevelTiles t{0, 0, 0, 0, 0};
+  if (lv.ok && bg.sub_log2 > 0) {
+    int side = bg.sub_log2;
+    // A level with few tasks of many candidates (a coarse level of a small call)
+    // takes 4 x 4 tiles, one MFMA sub-tile each: four times the tasks, each with
+    // about a third of the candidates, so that they do not run long after the other
+    // levels' tasks (the call waits for its longest task). K-blocks per 8 x 8 task,
+    // expected: 13 Q P / (10 * 64 * tiles).
+    if (bg.small_tiles) {
+      const int64_t t8 = int64_t((lv.w + 7) >> 3) * ((lv.h + 7) >> 3);
+      if (int64_t(p.B) * p.H * t8 < kSmallTileTasks &&
+          int64_t(p.Q) * p.P * 13 >= kSmallTileKBlocks * 10 * 64 * t8)
+        side = 2;
     }
-    lt[l] = t;
-    total += int64_t(t.ntx) * t.nty;
+    t.lw = t.lh = side;
+    t.ntx = (lv.w + (1 << t.lw) - 1) >> t.lw;
+    t.nty = (lv.h + (1 << t.lh) - 1) >> t.lh;
+  } else if (lv.ok) {
+    const int64_t records = 4 * int64_t(p.Q) * p.P;
+    const int64_t hw = int64_t(lv.h) * lv.w;
+    const int64_t want = records > 0 ? int64_t(kTargetRecords) * hw / records : bg.cap;
+    const int a = pow2_floor(std::min<int64_t>(std::max<int64_t>(want, bg.amin), bg.cap));
+    int tw0 = 1;
+    while (tw0 * tw0 < a) tw0 *= 2;
+    const int wcap = 1 << log2_ceil(lv.w), hcap = 1 << log2_ceil(lv.h);
+    int tw = min(wcap, tw0);
+    const int th = min(hcap, max(1, a / tw));
+    tw = min(wcap, max(tw, a / th));
+    t.lw = log2_ceil(tw);
+    t.lh = log2_ceil(th);
+    t.ntx = (lv.w + tw - 1) >> t.lw;
+    t.nty = (lv.h + th - 1) >> t.lh;
+  }
+  return t;
+}
+
+// Numbers the levels' tiles one after the other (one thread). Returns the tile count
+// of one (b, h), or -1 when it exceeds 2^29.
+__device__ inline int64_t number_tiles(int L, LevelTiles* lt) {
+  int64_t total = 0;
+  for (int l = 0; l < L; ++l) {
+    lt[l].base = int(total);
+    total += int64_t(lt[l].ntx) * lt[l].nty;
     if (total > (int64_t(1) << 29)) return -1;
   }
   return total;
@@ -972,7 +991,9 @@ __device__ inline int64_t load_tiles(const Problem& p, const BwdGeom& bg, Level*
   load_levels(p, levels);
   __syncthreads();
   overlap_flag_raise(levels, p.L);
-  if (threadIdx.x == 0) *total_out = plan_tiles(p, bg, levels, lt);
+  for (int l = threadIdx.x; l < p.L; l += blockDim.x) lt[l] = level_tiles(p, bg, levels[l]);
+  __syncthreads();
+  if (threadIdx.x == 0) *total_out = number_tiles(p.L, lt);
   __syncthreads();
   const bool any = *overlap_flag() != 0;
   if (overlap) *overlap = any;
@@ -1509,6 +1530,252 @@ __global__ __launch_bounds__(kSmallSortThreads) void msda_bucket_small_kernel(co
       for (int c = 0; c < 4; ++c)
         if (key[i][c] >= 0) out[slot[c]] = uint32_t(4 * (g0 + int64_t(i) * T) + c);
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The one-launch sort: records in bucket order, chunk by chunk.
+//
+// Workgroup (b, chunk, h) takes the samples of qc queries of one (b, h), at most
+// N = 4 GP blockDim.x of them: each thread loads GP groups of four samples of one
+// query and level (locations and weights, read once), the workgroup counts the
+// buckets in LDS (the rank of a sample in its bucket is what the atomic returns),
+// scans the counts, and moves the records through LDS into bucket order, so that
+// every stream is written with coalesced stores. A chunk is sorted by itself: no
+// count pass over the whole (b, h), no clear and no second pass over the locations;
+// the owner of a tile reads its range of every chunk instead of one range.
+//
+// Why: the counting sort over a whole (b, h) (clear, count, scan, place) reads the
+// locations, writes and re-reads a key per sample and scatters 4-byte entries (one L2
+// write request each), and the grad_value kernel then gathers every candidate's
+// location and weight through the entry: two requests per candidate and a dependent
+// load more. Here both are coalesced on both sides.
+//
+// Bucket order inside a tile: the samples that reach down only, those that reach
+// nowhere, those that reach right only, those that reach both ways. A tile's
+// candidates are then three contiguous ranges of a chunk: [left neighbour's samples
+// reaching right, the tile's own], [above-left's reaching both ways, above's reaching
+// down] and [above's reaching both ways]. (At the left edge the range starts in the
+// previous row's last tile, whose right-reaching buckets are empty.)
+constexpr int kRecordLevels = 16;   // levels at most
+constexpr int kRecordKeys = 4096;   // LDS bucket counters; more buckets take more passes
+constexpr size_t kRecordStaticLds = 18 * 1024;  // the sort's static LDS, at most
+constexpr int kRecordRanges = 3;    // ranges of a chunk a tile reads
+constexpr int kRecordGroup = kWave / kRecordRanges;  // chunks whose ranges one wave holds: 21
+// The calls it takes: at most this many samples per (query, head) (with softmax each
+// group of four forms the unit's softmax by itself), and positions per image (beyond,
+// the bucket passes would outnumber the rest of the sort).
+constexpr int64_t kRecordSamples = 1024;
+constexpr int64_t kRecordSoftmaxSamples = 64;
+constexpr int64_t kRecordPositions = int64_t(1) << 20;
+
+// The weight a record holds: as given, or (softmax) normalized, in float.
+template <typename T, bool SOFTMAX> using RecordWeight = std::conditional_t<SOFTMAX, float, T>;
+
+// Bucket of a sample for the record sort: 4 * tile + position of its sub-bucket.
+__device__ inline int record_bucket(int key) { return (key & ~3) | ((key + 1) & 3); }
+
+// The buckets of a chunk: four per tile (shift < 0), or, where the offsets of those do
+// not fit their memory (levels far from square, or overlapping ones: the host knows
+// only S and L), one per 2^shift consecutive tiles of a level. A tile then reads whole
+// buckets and ignores the samples that do not reach it.
+struct RecordBuckets {
+  int shift, count;
+};
+// Whole workgroup; `first` (shared) gets every level's first bucket. One barrier.
+__device__ inline RecordBuckets record_buckets(const Problem& p, const Records& r, const LevelTiles* lt,
+                                               int64_t ntiles, int* first) {
+  const int64_t rows = int64_t(p.B) * p.H * r.nch;
+  RecordBuckets b{-1, int(4 * ntiles)};
+  if (rows * (4 * ntiles + 1) > r.offs_cap) {
+    b.shift = 0;
+    while (rows * ((ntiles >> b.shift) + p.L + 1) > r.offs_cap && b.shift < 30) ++b.shift;
+  }
+  int at = 0;
+  for (int l = 0; l < p.L; ++l) {
+    const int nt = lt[l].ntx * lt[l].nty;
+    if (threadIdx.x == 0) first[l] = at;
+    at += b.shift < 0 ? 4 * nt : (nt + (1 << b.shift) - 1) >> b.shift;
+  }
+  b.count = at;
+  __syncthreads();
+  return b;
+}
+
+// One 4-sample group's raw locations.
+template <typename TL> struct GroupLoc {
+  u32x4_v w[2 * sizeof(TL) / 4];
+};
+
+template <typename T, typename TL, bool SOFTMAX, int GP>
+__global__ __launch_bounds__(1024) void msda_record_sort_kernel(const Problem p, const BwdGeom bg, const Records rec) {
+  using W = RecordWeight<T, SOFTMAX>;
+  using LocWord = std::conditional_t<sizeof(TL) == 2, uint32_t, u32x2_v>;  // one location pair
+  __shared__ Level levels[kRecordLevels];
+  __shared__ LevelTiles lt[kRecordLevels];
+  __shared__ int64_t total;
+  __shared__ int first[kRecordLevels];
+  __shared__ int hist[kRecordKeys];
+  __shared__ int scan_sums[1024 / kWave];
+  extern __shared__ __align__(16) unsigned char stage[];
+  const int T_ = int(blockDim.x), tid = int(threadIdx.x);
+  bool overlap = false;
+  const int64_t ntiles = load_tiles(p, bg, levels, lt, &total, &overlap);
+  if (overlap && p.zero_gv) zero_grad_value(p);
+  if (blockIdx.x == 0)
+    for (int i = tid; i < kXcds * kQueueLine; i += T_) rec.queue[i] = 0;
+  int group, h;
+  if (ntiles < 0 || !xcd_group_block(p.H, p.B * rec.nch, &group, &h)) return;
+  const int c = group % rec.nch, b = group / rec.nch;
+  const int LP = p.L * p.P, gpq = LP / 4;
+  const int q0 = c * rec.qc, nq = min(rec.qc, p.Q - q0);
+  const int ngroups = nq * gpq;
+  const int64_t unit0 = (int64_t(b) * p.Q + q0) * p.H + h;
+  const int64_t bh = int64_t(b) * p.H + h;
+  const RecordBuckets bk = record_buckets(p, rec, lt, ntiles, first);
+  const int nkeys = bk.count;
+
+  GroupLoc<TL> loc[GP];
+  W wt[GP][4];
+  int key[GP][4], pos[GP][4], ql[GP];
+#pragma unroll
+  for (int i = 0; i < GP; ++i) {
+    const int g = tid + i * T_;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) key[i][k] = pos[i][k] = -1;
+    ql[i] = 0;
+    if (g >= ngroups) continue;
+    const uint32_t q = fdiv(uint32_t(g), bg.div_gpq), r = uint32_t(g) - q * uint32_t(gpq);
+    ql[i] = int(q);
+    const int64_t unit = unit0 + int64_t(q) * p.H;
+    const u32x4_v* lc = reinterpret_cast<const u32x4_v*>(p.loc + (unit * LP + 4 * int(r)) * 2 * int64_t(sizeof(TL)));
+#pragma unroll
+    for (int k = 0; k < int(2 * sizeof(TL) / 4); ++k) loc[i].w[k] = lc[k];
+    const T* at = reinterpret_cast<const T*>(p.attn) + unit * LP;
+    if constexpr (SOFTMAX) {
+      // The unit's softmax, formed by each of its groups (the L P logits are
+      // neighbours in cache).
+      float mx = -INFINITY, sum = 0.f, a[4];
+      for (int j = 0; j < LP; j += 4) {
+        float v[4];
+        Chan<T, 4>::load(reinterpret_cast<const char*>(at + j), v);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) mx = fmax(mx, v[k]);
+      }
+      for (int j = 0; j < LP; j += 4) {
+        float v[4];
+        Chan<T, 4>::load(reinterpret_cast<const char*>(at + j), v);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sum += exp_acc(v[k] - mx);
+      }
+      const float lse = mx + log(sum);
+      Chan<T, 4>::load(reinterpret_cast<const char*>(at + 4 * int(r)), a);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) wt[i][k] = exp_acc(a[k] - lse);
+    } else {
+      const Raw<4 * sizeof(T)> a = *reinterpret_cast<const Raw<4 * sizeof(T)>*>(at + 4 * int(r));
+      __builtin_memcpy(wt[i], &a, sizeof(a));
+    }
+  }
+  auto pair_of = [&](const GroupLoc<TL>& l, int k) __attribute__((always_inline)) -> LocWord {
+    if constexpr (sizeof(TL) == 2) return l.w[0][k];
+    else return LocWord{l.w[k / 2][2 * (k & 1)], l.w[k / 2][2 * (k & 1) + 1]};
+  };
+#pragma unroll
+  for (int i = 0; i < GP; ++i) {
+    const int g = tid + i * T_;
+    if (g >= ngroups) continue;
+    const int l = int(fdiv(uint32_t(g) - uint32_t(ql[i]) * uint32_t(gpq), bg.div_gpl));
+    const Level lv = levels[l];
+    const LevelTiles tl = lt[l];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const LocWord v = pair_of(loc[i], k);
+      float x, y;
+      if constexpr (sizeof(TL) == 2) {
+        x = Chan16<TL, 2>::lo(v);
+        y = Chan16<TL, 2>::hi(v);
+      } else {
+        x = __uint_as_float(v[0]);
+        y = __uint_as_float(v[1]);
+      }
+      const int kk = sample_key<float>(x, y, lv, tl);
+      key[i][k] = kk < 0 ? -1 : bk.shift < 0 ? record_bucket(kk) : first[l] + ((kk / 4 - tl.base) >> bk.shift);
+    }
+  }
+
+  // Positions in bucket order, kRecordKeys buckets at a time.
+  uint16_t* row = rec.offs + (bh * rec.nch + c) * (int64_t(nkeys) + 1);
+  int base = 0;
+  for (int k0 = 0; k0 < nkeys; k0 += kRecordKeys) {
+    const int kn = min(kRecordKeys, nkeys - k0);
+    for (int k = tid; k < kn; k += T_) hist[k] = 0;
+    __syncthreads();
+    int kk[GP][4], slot[GP][4];
+#pragma unroll
+    for (int i = 0; i < GP; ++i) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int rel = key[i][k] - k0;
+        kk[i][k] = rel >= 0 && rel < kn ? rel : -1;
+      }
+      group_slots(kk[i], hist, slot[i]);
+    }
+    __syncthreads();
+    for (int s0 = 0; s0 < kn; s0 += T_) {
+      const int k = s0 + tid;
+      const int v = k < kn ? hist[k] : 0;
+      int sum;
+      const int ex = block_exclusive_scan(v, scan_sums, &sum);
+      if (k < kn) {
+        hist[k] = base + ex;
+        row[k0 + k] = uint16_t(base + ex);
+      }
+      base += sum;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < GP; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (slot[i][k] >= 0) pos[i][k] = hist[kk[i][k]] + slot[i][k];
+    __syncthreads();
+  }
+  if (tid == 0) row[nkeys] = uint16_t(base);
+
+  // The records through LDS: locations, then weights and queries. Whole groups of four
+  // records are copied (L P is a multiple of 4, so a region holds them).
+  const int n4 = (base + 3) >> 2;
+  const int64_t region = (bh * p.Q + q0) * LP;
+  LocWord* sl = reinterpret_cast<LocWord*>(stage);
+#pragma unroll
+  for (int i = 0; i < GP; ++i)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (pos[i][k] >= 0) sl[pos[i][k]] = pair_of(loc[i], k);
+  __syncthreads();
+  {
+    u32x4_v* dst = reinterpret_cast<u32x4_v*>(rec.loc + region * 2 * int64_t(sizeof(TL)));
+    for (int i = tid; i < n4 * int(2 * sizeof(TL) / 4); i += T_) dst[i] = reinterpret_cast<const u32x4_v*>(stage)[i];
+  }
+  __syncthreads();
+  W* sw = reinterpret_cast<W*>(stage);
+  uint16_t* sq = reinterpret_cast<uint16_t*>(stage + size_t(4 * GP) * T_ * sizeof(W));
+#pragma unroll
+  for (int i = 0; i < GP; ++i)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (pos[i][k] >= 0) {
+        sw[pos[i][k]] = wt[i][k];
+        sq[pos[i][k]] = uint16_t(ql[i]);
+      }
+  __syncthreads();
+  using Four = Raw<4 * sizeof(W)>;
+  Four* dw = reinterpret_cast<Four*>(rec.w + region * int64_t(sizeof(W)));
+  u32x2_v* dq = reinterpret_cast<u32x2_v*>(rec.q + region);
+  for (int i = tid; i < n4; i += T_) {
+    dw[i] = reinterpret_cast<const Four*>(sw)[i];
+    dq[i] = reinterpret_cast<const u32x2_v*>(sq)[i];
   }
 }
 
@@ -2117,7 +2384,9 @@ constexpr int kMfmaMaxNb = 4;     // 16-channel column blocks: D <= 64
 // a K-step has four sub-tiles of hi tiles, then four of lo tiles. A staged grad_out
 // row holds 16 nb 16-bit channels.
 constexpr int kMfmaWBytes = 16 * kMfmaKStep * 2;
-constexpr int kMfmaLoTiles = 4 * kMfmaWBytes;  // offset of the lo tiles
+constexpr int kMfmaSpare = 4 * kMfmaWBytes;  // a spare slot per lane after the hi tiles, for corners outside the tile
+constexpr int kMfmaLoTiles = kMfmaSpare + kWave * 2;  // offset of the lo tiles (and, after them, their spare slots)
+constexpr int kMfmaTileBytes = 2 * kMfmaLoTiles;
 constexpr int mfma_row_bytes(int nb) { return 16 * nb * 2; }
 // The MFMA operand type of a value dtype: f16 for f16 values, bf16 otherwise.
 template <typename T> constexpr bool mfma_f16_operands() { return std::is_same_v<T, f16_t>; }
@@ -2146,6 +2415,16 @@ __device__ inline void split_f16(float x, uint16_t* hi, uint16_t* lo) {
   const _Float16 r = static_cast<_Float16>(x - static_cast<float>(h));
   *lo = __builtin_isfinite(x) ? __builtin_bit_cast(uint16_t, r) : uint16_t(0);
 }
+// The parts of two finite weights, packed (b's in the high halves).
+template <bool F16> __device__ inline void split_pair(float a, float b, uint32_t* hi, uint32_t* lo) {
+  if constexpr (F16) {
+    *hi = pack_f16(a, b);
+    *lo = pack_f16(a - f16_bits(*hi & 0xffffu), b - f16_bits(*hi >> 16));
+  } else {
+    *hi = pack_bf16(a, b);
+    *lo = pack_bf16(a - bf16_lo(*hi), b - bf16_hi(*hi));
+  }
+}
 // Two floats to packed (hi, lo) bf16 pairs, element 0 in the low halves.
 __device__ inline void split_bf16_pair(float a, float b, uint32_t* hi, uint32_t* lo) {
   uint16_t ha, la, hb, lb;
@@ -2170,7 +2449,7 @@ size_t mfma_rows_bytes(int64_t D, bool split) {
   return size_t(kMfmaK) * size_t(mfma_row_bytes(int(D / 16))) * (split ? 2 : 1);
 }
 size_t mfma_wave_bytes(int64_t D, bool split) {
-  const size_t work = mfma_rows_bytes(D, split) + 8 * size_t(kMfmaWBytes);
+  const size_t work = mfma_rows_bytes(D, split) + size_t(kMfmaTileBytes);
   const size_t partial = 4 * size_t(D / 16) * kWave * 16;
   return std::max(work, partial);
 }
@@ -2238,15 +2517,6 @@ __device__ inline uint32_t cand_entry(const uint32_t* __restrict__ ent, const Ca
   return ent[c + off];
 }
 
-// One K-block's loads for one lane: its candidate's location and weight (MfmaMeta,
-// loaded a block ahead), and its share of the block's grad_out rows (MfmaRows: flat
-// 16-byte piece lane + 64 j of the 64 rows, loaded half a block ahead, as soon as
-// the previous block has staged its rows).
-template <typename T, typename TL> struct MfmaMeta {
-  LocPair<TL> loc;
-  T attn;              // the weight, or with softmax the logit
-  SoftStat<float> st;  // softmax: the unit's statistics (when stats are kept)
-};
 template <int NP> struct MfmaRows {
   u32x4_v piece[NP];
 };
@@ -2255,32 +2525,155 @@ template <typename T, int NB> constexpr int mfma_pieces() { return NB * int(size
 
 // Per-tile constants of the matrix-core kernel (all wave-uniform).
 struct MfmaTile {
-  const char* loc;   // locations of (b, q = 0, h)
-  const char* attn;  // weights of (b, q = 0, h)
-  const char* gout;  // grad_out row of (b, q = 0, h)
-  uint32_t loc_q, attn_q, gout_q;  // bytes per query step
-  int r0, c0, r1, c1;              // tile rows [r0, r1), columns [c0, c1)
-  int nst;                         // sub-tiles the tile has: 4 (8 x 8), or 1 (4 x 4)
-  uint32_t ncand;
-  FastDiv div_lp;
-  int LP;
-  const SoftStat<float>* stats;  // softmax statistics of (b, q = 0, h), stride H per query; or null
-  int H;
+  const char* gout;    // grad_out row of (b, q = 0, h)
+  uint32_t gout_q;     // bytes per query step
+  int r0, c0, r1, c1;  // tile rows [r0, r1), columns [c0, c1)
+  int nst;             // sub-tiles the tile has: 4 (8 x 8), or 1 (4 x 4)
 };
 
-template <typename T, typename TL, bool SOFTMAX>
-__device__ inline void mfma_load_meta(const MfmaTile& t, uint32_t e, MfmaMeta<T, TL>& d) {
-  const uint32_t q = fdiv(e, t.div_lp), s = e - q * uint32_t(t.LP);
-  d.loc = *reinterpret_cast<const LocPair<TL>*>(t.loc + (__umul24(q, t.loc_q) + s * uint32_t(2 * sizeof(TL))));
-  if (!SOFTMAX || t.stats) d.attn = *reinterpret_cast<const T*>(t.attn + (__umul24(q, t.attn_q) + s * uint32_t(sizeof(T))));
-  if constexpr (SOFTMAX)
-    if (t.stats) d.st = t.stats[__umul24(q, uint32_t(t.H))];
-}
+// Where a tile's candidates come from. A source hands out, for a lane's candidate of a
+// K-block (64 candidates from number `first` on; past the end any valid one):
+//   ref(first)     its handle, with the first of its loads (two K-blocks ahead),
+//   meta(ref)      its location and weight loads (one K-block ahead),
+//   query(ref)     its query, for the grad_out rows,
+//   weight(ref, m) its attention weight.
+// ncand: how many there are.
+
+// Candidates from the counting sort's entries: sample indices, through which location
+// and weight (with softmax the logit and, when kept, the unit's statistics) are gathered.
+template <typename T, typename TL, bool SOFTMAX> struct EntrySource {
+  const uint32_t* ent;
+  CandRanges cr;
+  const char* loc;   // locations of (b, q = 0, h)
+  const char* attn;  // weights of (b, q = 0, h)
+  uint32_t loc_q, attn_q;  // bytes per query step
+  FastDiv div_lp;
+  int LP, H;
+  const SoftStat<float>* stats;  // softmax statistics of (b, q = 0, h), stride H per query; or null
+  uint32_t ncand;
+  int lane;
+
+  using Ref = uint32_t;
+  struct Meta {
+    LocPair<TL> loc;
+    T attn;
+    SoftStat<float> st;
+  };
+  __device__ inline Ref ref(uint32_t first) const { return cand_entry(ent, cr, first + uint32_t(lane)); }
+  __device__ inline uint32_t query(Ref e) const { return fdiv(e, div_lp); }
+  __device__ inline void meta(Ref e, Meta& d) const {
+    const uint32_t q = fdiv(e, div_lp), s = e - q * uint32_t(LP);
+    d.loc = *reinterpret_cast<const LocPair<TL>*>(loc + (__umul24(q, loc_q) + s * uint32_t(2 * sizeof(TL))));
+    if (!SOFTMAX || stats) d.attn = *reinterpret_cast<const T*>(attn + (__umul24(q, attn_q) + s * uint32_t(sizeof(T))));
+    if constexpr (SOFTMAX)
+      if (stats) d.st = stats[__umul24(q, uint32_t(H))];
+  }
+  __device__ inline float weight(Ref e, const Meta& d) const {
+    if constexpr (SOFTMAX) {
+      if (stats) return exp_acc(to_acc(d.attn) - d.st.lse);
+      const uint32_t q = fdiv(e, div_lp), s = e - q * uint32_t(LP);
+      return unit_weight<T, true>(reinterpret_cast<const T*>(attn + __umul24(q, attn_q)), LP, int(s));
+    } else {
+      return to_acc(d.attn);
+    }
+  }
+};
+
+// Candidates from the record streams: a tile's ranges of up to kRecordGroup chunks,
+// one range per lane. Candidate numbers run through the ranges in lane order.
+template <typename T, typename TL, bool SOFTMAX> struct RecordSource {
+  using W = RecordWeight<T, SOFTMAX>;
+  const char* loc;      // the streams at (b, h)
+  const W* w;
+  const uint16_t* q;
+  const uint16_t* offs;  // the offsets of (b, h), chunk 0
+  uint32_t row;         // offsets per chunk
+  int nch, qc, LP;
+  int g0;               // first chunk of the group in hand
+  uint32_t pre, n;      // this lane's range: candidates before it, and in it
+  uint32_t delta;       // record of its candidate j: j + delta
+  uint32_t ncand;
+  int* slots;           // kWave ints of the wave's LDS
+  int lane;
+
+  struct Ref {
+    uint32_t idx, q0;
+    uint16_t ql;
+  };
+  struct Meta {
+    LocPair<TL> loc;
+    W w;
+  };
+
+  // Takes the ranges of the chunks from g on: tile `tile`, in tile row ty, of a level
+  // whose first bucket is `kb`.
+  __device__ inline void group(int g, uint32_t kb, int tile, int ntx, int ty, int shift) {
+    g0 = g;
+    const int kind = lane / kRecordGroup, c = g + lane - kind * kRecordGroup;
+    uint32_t s0 = 0, s1 = 0;
+    if (kind < kRecordRanges && c < nch && (kind == 0 || ty > 0)) {
+      const int u = tile - ntx;
+      int k0, k1;
+      if (shift >= 0) {  // the buckets of this tile and its left neighbour, then (once) those of the two above
+        const int own = max(tile - 1, 0) >> shift;
+        k0 = kind == 0 ? own : max(u - 1, 0) >> shift;
+        k1 = kind == 0 ? (tile >> shift) + 1 : kind == 1 ? min((u >> shift) + 1, own) : k0;
+        k1 = max(k0, k1);
+      } else if (kind == 0) {
+        k0 = tile > 0 ? 4 * tile - 2 : 0;
+        k1 = 4 * tile + 4;
+      } else {
+        k0 = kind == 1 ? (u > 0 ? 4 * u - 1 : 0) : 4 * u + 3;
+        k1 = kind == 1 ? 4 * u + 1 : 4 * u + 4;
+      }
+      const uint16_t* o = offs + uint32_t(c) * row + kb;
+      s0 = o[k0];
+      s1 = o[k1];
+    }
+    n = s1 - s0;
+    const int inc = wave_inclusive_scan(int(n));
+    pre = uint32_t(inc) - n;
+    ncand = uint32_t(__builtin_amdgcn_readlane(inc, kWave - 1));
+    delta = uint32_t(c) * uint32_t(qc * LP) + s0 - pre;
+  }
+  // The range of candidate number first + lane: the last non-empty one that starts at or
+  // before it. Ranges that start inside the block mark their first candidate's slot with
+  // their lane; a running maximum over the lanes spreads the marks.
+  __device__ inline Ref ref(uint32_t first) const {
+    const uint32_t rel = pre - first;  // beyond 64 also when the range starts before `first`
+    wave_lds_order();
+    slots[lane] = 0;
+    wave_lds_order();
+    if (n > 0 && pre > first && rel < uint32_t(kWave)) slots[rel] = lane;
+    wave_lds_order();
+    const uint64_t before = __ballot(n > 0 && pre <= first);
+    const int seed = before ? 63 - __builtin_clzll(before) : 0;
+    int v = slots[lane];
+    if (lane == 0) v = seed;
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+    Ref r;
+    r.idx = min(first + uint32_t(lane), ncand - 1) + uint32_t(__shfl(int(delta), v));
+    const int kind = v / kRecordGroup;
+    r.q0 = uint32_t(g0 + v - kind * kRecordGroup) * uint32_t(qc);
+    r.ql = q[r.idx];
+    return r;
+  }
+  __device__ inline uint32_t query(const Ref& r) const { return r.q0 + r.ql; }
+  __device__ inline void meta(const Ref& r, Meta& d) const {
+    d.loc = *reinterpret_cast<const LocPair<TL>*>(loc + r.idx * uint32_t(2 * sizeof(TL)));
+    d.w = w[r.idx];
+  }
+  __device__ inline float weight(const Ref&, const Meta& d) const { return to_acc(d.w); }
+};
 
 template <typename T, int NB>
-__device__ inline void mfma_load_rows(const MfmaTile& t, uint32_t e, int lane, MfmaRows<mfma_pieces<T, NB>()>& d) {
+__device__ inline void mfma_load_rows(const MfmaTile& t, uint32_t q, int lane, MfmaRows<mfma_pieces<T, NB>()>& d) {
   constexpr int kPieces = mfma_pieces<T, NB>();  // 16-byte pieces per grad_out row
-  const uint32_t q = fdiv(e, t.div_lp);
 #pragma unroll
   for (int j = 0; j < kPieces; ++j) {
     const int f = lane + kWave * j, row = f / kPieces, pc = f - row * kPieces;
@@ -2300,8 +2693,8 @@ __device__ inline void mfma_load_rows(const MfmaTile& t, uint32_t e, int lane, M
 // far less LDS bandwidth than zeroing the 8 KB of tiles per K-step. A wave's LDS
 // instructions execute in order, so the clears land after the operand reads.
 struct MfmaCorners {
-  int o[4];
-  uint16_t hi[4], lo[4];
+  uint32_t o[4];
+  uint32_t hi[2], lo[2];  // parts of corners (0, 1) and (2, 3), the first in the low half
 };
 
 // A staged 16-byte piece of a grad_out row: copied (bf16, f16), or split into bf16
@@ -2324,62 +2717,55 @@ __device__ inline void mfma_stage_piece(const u32x4_v& v, unsigned char* hi, uns
   }
 }
 
-template <typename T, typename TL, int NB, bool SOFTMAX>
-__device__ inline MfmaCorners mfma_kblock_a(const MfmaTile& t, const Level& lv, uint32_t kb, uint32_t e,
-                                            const MfmaMeta<T, TL>& d, const MfmaRows<mfma_pieces<T, NB>()>& rows,
-                                            int lane, unsigned char* gst) {
+template <typename T, int NB, typename Source>
+__device__ inline MfmaCorners mfma_kblock_a(const Source& src, const MfmaTile& t, const Level& lv, uint32_t kb,
+                                            const typename Source::Ref& e, const typename Source::Meta& d,
+                                            const MfmaRows<mfma_pieces<T, NB>()>& rows, int lane,
+                                            unsigned char* gst) {
   constexpr int ES = int(sizeof(T));
   constexpr int kPieces = mfma_pieces<T, NB>();
   constexpr int kRowBytes = mfma_row_bytes(NB);
   constexpr int kStagedPiece = 16 * 2 / ES;  // staged bytes a 16-byte piece becomes
   constexpr size_t kLoRows = size_t(kMfmaK) * kRowBytes;
-  const int kc = lane & (kMfmaKStep - 1);
-  const uint32_t c = kb * kMfmaK + uint32_t(lane);
+  // The candidate's corners in the tile, without branches: a corner outside it (or of a
+  // lane past the end) goes to the lane's own spare slot. Every candidate is in range of
+  // the level, and the tile's bounds are inside it.
   MfmaCorners cr;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    cr.o[k] = -1;
-    cr.hi[k] = cr.lo[k] = 0;
+  {
+#pragma clang fp contract(off)
+    const float x = to_acc(d.loc.x) * float(lv.w) - 0.5f, y = to_acc(d.loc.y) * float(lv.h) - 0.5f;
+    const float xf = floor(x), yf = floor(y);
+    const float dx = x - xf, dy = y - yf;
+    const uint32_t x0 = uint32_t(int(xf) - t.c0), y0 = uint32_t(int(yf) - t.r0);
+    const uint32_t x1 = x0 + 1, y1 = y0 + 1;
+    const uint32_t nx = uint32_t(t.c1 - t.c0);
+    const uint32_t ny = kb * kMfmaK + uint32_t(lane) < src.ncand ? uint32_t(t.r1 - t.r0) : 0u;
+    // Position (y, x) of the tile: sub-tile (y / 4) * 2 + x / 4, row (y % 4) * 4 + x % 4
+    // of its position-major [16][32] weight tile.
+    const uint32_t kc = uint32_t(lane & (kMfmaKStep - 1)) * 2;
+    auto xo = [](uint32_t v) { return (v >> 2) * kMfmaWBytes + (v & 3) * (2 * kMfmaKStep); };
+    auto yo = [](uint32_t v) { return (v >> 2) * (2 * kMfmaWBytes) + (v & 3) * (8 * kMfmaKStep); };
+    const uint32_t xo0 = xo(x0) + kc, xo1 = xo(x1) + kc, yo0 = yo(y0), yo1 = yo(y1);
+    const uint32_t spare = uint32_t(kMfmaSpare + lane * 2);
+    cr.o[0] = y0 < ny && x0 < nx ? yo0 + xo0 : spare;
+    cr.o[1] = y0 < ny && x1 < nx ? yo0 + xo1 : spare;
+    cr.o[2] = y1 < ny && x0 < nx ? yo1 + xo0 : spare;
+    cr.o[3] = y1 < ny && x1 < nx ? yo1 + xo1 : spare;
+    const float a = src.weight(e, d);
+    const float ex = 1.f - dx, ey = 1.f - dy;
+    split_pair<mfma_f16_operands<T>()>(ex * ey * a, dx * ey * a, &cr.hi[0], &cr.lo[0]);
+    split_pair<mfma_f16_operands<T>()>(ex * dy * a, dx * dy * a, &cr.hi[1], &cr.lo[1]);
+    // The weights are as finite as the attention weight; the low parts of non-finite
+    // ones are zero.
+    if (!__builtin_isfinite(a)) cr.lo[0] = cr.lo[1] = 0;
   }
-  if (c < t.ncand) {
-    const Geom<float> g = geometry<float>(to_acc(d.loc.x), to_acc(d.loc.y), lv, 0u, 1u);
-    float a;
-    if constexpr (SOFTMAX) {
-      if (t.stats) {
-        a = exp_acc(to_acc(d.attn) - d.st.lse);
-      } else {
-        const uint32_t q = fdiv(e, t.div_lp), s = e - q * uint32_t(t.LP);
-        a = unit_weight<T, true>(reinterpret_cast<const T*>(t.attn + __umul24(q, t.attn_q)), t.LP, int(s));
-      }
-    } else {
-      a = to_acc(d.attn);
-    }
-    const bool m[4] = {g.m00, g.m01, g.m10, g.m11};
-    const float wb[4] = {g.w00, g.w01, g.w10, g.w11};
-    const int y0 = g.iy - t.r0, x0 = g.ix - t.c0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int y = y0 + (k >> 1), x = x0 + (k & 1);
-      // Position (y, x) of the tile: sub-tile (y / 4) * 2 + x / 4, row (y % 4) * 4 + x % 4
-      // of its position-major [16][32] weight tile.
-      if (m[k] && y >= 0 && x >= 0 && t.r0 + y < t.r1 && t.c0 + x < t.c1) {
-        const int pos = (y & 3) * 4 + (x & 3);
-        cr.o[k] = ((y >> 2) * 2 + (x >> 2)) * kMfmaWBytes + pos * (2 * kMfmaKStep) + kc * 2;
-        if constexpr (mfma_f16_operands<T>())
-          split_f16(wb[k] * a, &cr.hi[k], &cr.lo[k]);
-        else
-          split_bf16(wb[k] * a, &cr.hi[k], &cr.lo[k]);
-      }
-    }
-  }
+  // Rows past the end repeat a candidate's (their weights are zero).
   wave_lds_order();  // after the previous K-block's operand reads
-  const u32x4_v zero = {0u, 0u, 0u, 0u};
 #pragma unroll
   for (int j = 0; j < kPieces; ++j) {
     const int f = lane + kWave * j, row = f / kPieces, pc = f - row * kPieces;
-    const bool ok = kb * kMfmaK + uint32_t(row) < t.ncand;  // past the end: zero rows
     unsigned char* dst = gst + row * kRowBytes + pc * kStagedPiece;
-    mfma_stage_piece<T>(ok ? rows.piece[j] : zero, dst, dst + kLoRows);
+    mfma_stage_piece<T>(rows.piece[j], dst, dst + kLoRows);
   }
   return cr;
 }
@@ -2401,11 +2787,10 @@ __device__ inline void mfma_kblock_b(const MfmaCorners& cr, int lane, const unsi
     wave_lds_order();
     if (half == ks) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (cr.o[k] >= 0) {
-          *reinterpret_cast<uint16_t*>(wt + cr.o[k]) = cr.hi[k];
-          *reinterpret_cast<uint16_t*>(wt + kMfmaLoTiles + cr.o[k]) = cr.lo[k];
-        }
+      for (int k = 0; k < 4; ++k) {
+        *reinterpret_cast<uint16_t*>(wt + cr.o[k]) = uint16_t(cr.hi[k / 2] >> (16 * (k & 1)));
+        *reinterpret_cast<uint16_t*>(wt + kMfmaLoTiles + cr.o[k]) = uint16_t(cr.lo[k / 2] >> (16 * (k & 1)));
+      }
     }
     wave_lds_order();
     u32x4_v bh[NB], bl[NB];
@@ -2435,11 +2820,10 @@ __device__ inline void mfma_kblock_b(const MfmaCorners& cr, int lane, const unsi
     wave_lds_order();
     if (half == ks) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (cr.o[k] >= 0) {
-          *reinterpret_cast<uint16_t*>(wt + cr.o[k]) = 0;
-          *reinterpret_cast<uint16_t*>(wt + kMfmaLoTiles + cr.o[k]) = 0;
-        }
+      for (int k = 0; k < 4; ++k) {
+        *reinterpret_cast<uint16_t*>(wt + cr.o[k]) = 0;
+        *reinterpret_cast<uint16_t*>(wt + kMfmaLoTiles + cr.o[k]) = 0;
+      }
     }
   }
 }
@@ -2450,71 +2834,64 @@ __device__ inline void mfma_zero_tiles(unsigned char* wt, int lane) {
   const u32x4_v zero = {0u, 0u, 0u, 0u};
   wave_lds_order();
 #pragma unroll
-  for (int z = 0; z < 8 * kMfmaWBytes / (kWave * 16); ++z)
+  for (int z = 0; z < 4 * kMfmaWBytes / (kWave * 16); ++z) {
     *reinterpret_cast<u32x4_v*>(wt + (z * kWave + lane) * 16) = zero;
+    *reinterpret_cast<u32x4_v*>(wt + kMfmaLoTiles + (z * kWave + lane) * 16) = zero;
+  }
   wave_lds_order();
 }
 
 // K-steps of K-block kb that hold candidates (the rest would add zeros).
-__device__ inline int mfma_ksteps(const MfmaTile& t, uint32_t kb) {
-  return t.ncand > kb * kMfmaK + kMfmaKStep ? 2 : 1;
+__device__ inline int mfma_ksteps(uint32_t ncand, uint32_t kb) {
+  return ncand > kb * kMfmaK + kMfmaKStep ? 2 : 1;
 }
 
-// The K-blocks kb0, kb0 + kbstep, ... of one tile into acc (zeroed here). Block j's
-// entries are loaded two blocks ahead, its locations and weights one block ahead
+// Adds the K-blocks kb0, kb0 + kbstep, ... of a source's candidates into acc. Block j's
+// refs are loaded two blocks ahead, its locations and weights one block ahead
 // (two register sets in turn) and its grad_out rows as soon as block j - 1 has
 // staged its own, each before the loads of later blocks, so that a wait for one
 // never waits for younger loads. The main loop issues its loads unconditionally
-// (an entry past the end reads candidate 0), so that the compiler's wait counts
+// (a candidate past the end reads a valid one), so that the compiler's wait counts
 // stay exact; the last one or two blocks run after it.
-template <typename T, typename TL, int NB, bool SOFTMAX, int NST>
-__device__ inline void mfma_tile_kblocks(const MfmaTile& t, const Level& lv, const CandRanges& cr,
-                                         const uint32_t* __restrict__ ent, int kb0, int kbstep, int lane,
-                                         unsigned char* gst, unsigned char* wt, f32x4_v (&acc)[4][NB]) {
-#pragma unroll
-  for (int st = 0; st < 4; ++st)
-#pragma unroll
-    for (int j = 0; j < NB; ++j) acc[st][j] = f32x4_v{0.f, 0.f, 0.f, 0.f};
-  const uint32_t nkb = (cr.ncand + kMfmaK - 1) / kMfmaK;
+template <typename T, int NB, int NST, typename Source>
+__device__ inline void mfma_tile_kblocks(const Source& src, const MfmaTile& t, const Level& lv, int kb0, int kbstep,
+                                         int lane, unsigned char* gst, unsigned char* wt, f32x4_v (&acc)[4][NB]) {
+  const uint32_t nkb = (src.ncand + kMfmaK - 1) / kMfmaK;
   const uint32_t mine = nkb > uint32_t(kb0) ? (nkb - uint32_t(kb0) + uint32_t(kbstep) - 1) / uint32_t(kbstep) : 0u;
+  if (mine == 0) return;
   const uint32_t step = uint32_t(kbstep) * kMfmaK;
-  uint32_t cand = uint32_t(kb0) * kMfmaK + uint32_t(lane);  // this lane's candidate in block j
-  MfmaMeta<T, TL> ma, mb;
+  uint32_t cand = uint32_t(kb0) * kMfmaK;  // first candidate of block j
+  typename Source::Meta ma, mb;
   MfmaRows<mfma_pieces<T, NB>()> rows;
-  uint32_t ea = 0, eb = 0, j = 0;
-  if (mine > 0) {
-    ea = cand_entry(ent, cr, cand);
-    eb = cand_entry(ent, cr, cand + step);
-    mfma_load_meta<T, TL, SOFTMAX>(t, ea, ma);
-    mfma_load_rows<T, NB>(t, ea, lane, rows);
-  }
+  uint32_t j = 0;
+  typename Source::Ref ea = src.ref(cand), eb = src.ref(cand + step);
+  src.meta(ea, ma);
+  mfma_load_rows<T, NB>(t, src.query(ea), lane, rows);
   for (; j + 2 < mine; j += 2) {
     const uint32_t kb = uint32_t(kb0) + j * uint32_t(kbstep);
-    const uint32_t e2 = cand_entry(ent, cr, cand + 2 * step);
-    mfma_load_meta<T, TL, SOFTMAX>(t, eb, mb);
-    const auto c0 = mfma_kblock_a<T, TL, NB, SOFTMAX>(t, lv, kb, ea, ma, rows, lane, gst);
-    mfma_load_rows<T, NB>(t, eb, lane, rows);
+    const typename Source::Ref e2 = src.ref(cand + 2 * step);
+    src.meta(eb, mb);
+    const auto c0 = mfma_kblock_a<T, NB>(src, t, lv, kb, ea, ma, rows, lane, gst);
+    mfma_load_rows<T, NB>(t, src.query(eb), lane, rows);
     mfma_kblock_b<T, NB, NST>(c0, lane, gst, wt, acc);
-    const uint32_t e3 = cand_entry(ent, cr, cand + 3 * step);
-    mfma_load_meta<T, TL, SOFTMAX>(t, e2, ma);
-    const auto c1 = mfma_kblock_a<T, TL, NB, SOFTMAX>(t, lv, kb + uint32_t(kbstep), eb, mb, rows, lane, gst);
-    mfma_load_rows<T, NB>(t, e2, lane, rows);
+    const typename Source::Ref e3 = src.ref(cand + 3 * step);
+    src.meta(e2, ma);
+    const auto c1 = mfma_kblock_a<T, NB>(src, t, lv, kb + uint32_t(kbstep), eb, mb, rows, lane, gst);
+    mfma_load_rows<T, NB>(t, src.query(e2), lane, rows);
     mfma_kblock_b<T, NB, NST>(c1, lane, gst, wt, acc);
     ea = e2;
     eb = e3;
     cand += 2 * step;
   }
-  if (j < mine) {
-    const uint32_t kb = uint32_t(kb0) + j * uint32_t(kbstep);
-    const bool two = j + 1 < mine;
-    if (two) mfma_load_meta<T, TL, SOFTMAX>(t, eb, mb);
-    const auto c0 = mfma_kblock_a<T, TL, NB, SOFTMAX>(t, lv, kb, ea, ma, rows, lane, gst);
-    if (two) mfma_load_rows<T, NB>(t, eb, lane, rows);
-    mfma_kblock_b<T, NB, NST, true>(c0, lane, gst, wt, acc, mfma_ksteps(t, kb));
-    if (two) {
-      const auto c1 = mfma_kblock_a<T, TL, NB, SOFTMAX>(t, lv, kb + uint32_t(kbstep), eb, mb, rows, lane, gst);
-      mfma_kblock_b<T, NB, NST, true>(c1, lane, gst, wt, acc, mfma_ksteps(t, kb + uint32_t(kbstep)));
-    }
+  const uint32_t kb = uint32_t(kb0) + j * uint32_t(kbstep);
+  const bool two = j + 1 < mine;
+  if (two) src.meta(eb, mb);
+  const auto c0 = mfma_kblock_a<T, NB>(src, t, lv, kb, ea, ma, rows, lane, gst);
+  if (two) mfma_load_rows<T, NB>(t, src.query(eb), lane, rows);
+  mfma_kblock_b<T, NB, NST, true>(c0, lane, gst, wt, acc, mfma_ksteps(src.ncand, kb));
+  if (two) {
+    const auto c1 = mfma_kblock_a<T, NB>(src, t, lv, kb + uint32_t(kbstep), eb, mb, rows, lane, gst);
+    mfma_kblock_b<T, NB, NST, true>(c1, lane, gst, wt, acc, mfma_ksteps(src.ncand, kb + uint32_t(kbstep)));
   }
 }
 
@@ -2613,15 +2990,19 @@ __device__ inline int region_first_tile(int r, int n, int extent, int ntiles, in
 // early takes the next task of its queue. A small LDS table of prefix counts per
 // (pair, level) maps a queue position to its task. When the table would not fit,
 // queue x holds the x-th eighth of each level's tasks (b, tile, h) in raster order.
-template <typename T, typename TL, int NB, bool SOFTMAX>
+// RECORDS: the candidates come from the record streams; else from `buckets` and
+// `entries`.
+template <typename T, typename TL, int NB, bool SOFTMAX, bool RECORDS>
 __global__ __launch_bounds__(kWave * kMfmaWaves, mfma_blocks_per_cu(NB, int(sizeof(T)))) void msda_grad_value_mfma_kernel(
     const Problem p, const BwdGeom bg, int* __restrict__ buckets,
-    const uint32_t* __restrict__ entries, const int accumulate, const int table_cap) {
+    const uint32_t* __restrict__ entries, const Records rec, const int accumulate, const int table_cap) {
   constexpr int D = 16 * NB;
   constexpr int ES = int(sizeof(T));
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int wave_sums[kMfmaWaves];
   __shared__ int grid_s[2];
+  __shared__ int slots_s[RECORDS ? kMfmaWaves : 1][kWave];
+  __shared__ int level_buckets[RECORDS ? kRecordLevels : 1];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const int LP = p.L * p.P;
 
@@ -2641,7 +3022,7 @@ __global__ __launch_bounds__(kWave * kMfmaWaves, mfma_blocks_per_cu(NB, int(size
   at += 16;
   constexpr bool kSplit = sizeof(T) == 4;
   constexpr size_t kRowsBytes = size_t(kMfmaK) * size_t(mfma_row_bytes(NB)) * (kSplit ? 2 : 1);
-  constexpr size_t kWaveBytes = std::max(kRowsBytes + 8 * size_t(kMfmaWBytes), size_t(4 * NB * kWave * 16));
+  constexpr size_t kWaveBytes = std::max(kRowsBytes + size_t(kMfmaTileBytes), size_t(4 * NB * kWave * 16));
   unsigned char* region0 = smem + at;
   unsigned char* gst = region0 + size_t(wave) * kWaveBytes;  // grad_out rows (hi, then lo)
   unsigned char* wt = gst + kRowsBytes;                      // eight weight tiles (hi, then lo)
@@ -2671,8 +3052,10 @@ __global__ __launch_bounds__(kWave * kMfmaWaves, mfma_blocks_per_cu(NB, int(size
       }
     }
   }
-  if (ntiles <= 0 || !queue_fits(p, bg, 4 * ntiles)) return;  // the VALU owner kernel runs instead
-  const bool stats_ok = SOFTMAX && (p.stats || softmax_stats_fit<float>(p, bg, 4 * ntiles, buckets));
+  if (ntiles <= 0 || (!RECORDS && !queue_fits(p, bg, 4 * ntiles))) return;  // the VALU owner kernel runs instead
+  RecordBuckets bk{};
+  if constexpr (RECORDS) bk = record_buckets(p, rec, lt, ntiles, level_buckets);
+  const bool stats_ok = SOFTMAX && !RECORDS && (p.stats || softmax_stats_fit<float>(p, bg, 4 * ntiles, buckets));
   if (tid == 0) {
     order_levels(p, levels, lt, order, rank_base);
     // R x R regions, R the power of two nearest the finest level's tile count, at most
@@ -2703,9 +3086,10 @@ __global__ __launch_bounds__(kWave * kMfmaWaves, mfma_blocks_per_cu(NB, int(size
   __syncthreads();
 
   const int xcd = int(blockIdx.x) % kXcds;
-  int* queue = reinterpret_cast<int*>(
-                   (reinterpret_cast<uintptr_t>(buckets + int64_t(p.B) * p.H * 4 * ntiles) + 4 * kQueueLine - 1) &
-                   ~uintptr_t(4 * kQueueLine - 1)) +
+  int* queue = (RECORDS ? rec.queue
+                        : reinterpret_cast<int*>((reinterpret_cast<uintptr_t>(buckets + int64_t(p.B) * p.H * 4 * ntiles) +
+                                                  4 * kQueueLine - 1) &
+                                                 ~uintptr_t(4 * kQueueLine - 1))) +
                xcd * kQueueLine;
   const int64_t per_tile = int64_t(p.B) * p.H;
   const int R = grid_s[0];  // regions per axis, a power of two; visited in Morton order
@@ -2843,37 +3227,68 @@ __global__ __launch_bounds__(kWave * kMfmaWaves, mfma_blocks_per_cu(NB, int(size
       tl = LevelTiles{uni(tl.lh), uni(tl.lw), uni(tl.ntx), uni(tl.nty), uni(tl.base)};
       const int ty = tile / tl.ntx, tx = tile - ty * tl.ntx;
       const int bh = b * p.H + h;
-      const uint32_t* ent = entries + int64_t(bh) * bg.region;
-      const CandRanges cr = tile_candidates(buckets + int64_t(bh) * 4 * ntiles, tl, tile, tx, ty, uint32_t(l * p.P));
       const int64_t unit0 = int64_t(b) * p.Q * p.H + h;  // (b, q = 0, h)
       MfmaTile t;
-      t.loc = p.loc + unit0 * LP * 2 * int64_t(sizeof(TL));
-      t.attn = p.attn + unit0 * LP * ES;
       t.gout = p.grad_out + unit0 * D * ES;
-      t.loc_q = uint32_t(p.H * LP * 2) * uint32_t(sizeof(TL));
-      t.attn_q = uint32_t(p.H * LP * ES);
       t.gout_q = uint32_t(p.H * D * ES);
       t.r0 = ty << tl.lh;
       t.c0 = tx << tl.lw;
       t.r1 = min(t.r0 + (1 << tl.lh), lv.h);
       t.c1 = min(t.c0 + (1 << tl.lw), lv.w);
       t.nst = tl.lw < kMfmaSubLog2 ? 1 : 4;  // a 4 x 4 tile is sub-tile 0 alone
-      t.ncand = cr.ncand;
-      t.div_lp = bg.div_lp;
-      t.LP = LP;
-      t.H = p.H;
-      t.stats = SOFTMAX && stats_ok ? (p.stats ? reinterpret_cast<const SoftStat<float>*>(p.stats)
-                                               : softmax_stats<float>(buckets, p, 4 * ntiles)) + unit0
-                                    : nullptr;
 
       f32x4_v acc[4][NB];
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[st][j] = f32x4_v{0.f, 0.f, 0.f, 0.f};
       // All K-blocks (per-wave mode), or K-blocks wave, wave + 4, ...
-      if (t.nst == 1)  // wave-uniform: a 4 x 4 tile runs one sub-tile's MFMAs
-        mfma_tile_kblocks<T, TL, NB, SOFTMAX, 1>(t, lv, cr, ent, per_wave ? 0 : wave, per_wave ? 1 : kMfmaWaves,
-                                                 lane, gst, wt, acc);
-      else
-        mfma_tile_kblocks<T, TL, NB, SOFTMAX, 4>(t, lv, cr, ent, per_wave ? 0 : wave, per_wave ? 1 : kMfmaWaves,
-                                                 lane, gst, wt, acc);
+      const int kb0 = per_wave ? 0 : wave, kbstep = per_wave ? 1 : kMfmaWaves;
+      if constexpr (RECORDS) {
+        RecordSource<T, TL, SOFTMAX> src;
+        src.row = uint32_t(bk.count + 1);
+        const int64_t first = int64_t(bh) * p.Q * LP;
+        src.loc = rec.loc + first * 2 * int64_t(sizeof(TL));
+        src.w = reinterpret_cast<const RecordWeight<T, SOFTMAX>*>(rec.w) + first;
+        src.q = rec.q + first;
+        src.offs = rec.offs + int64_t(bh) * rec.nch * src.row;
+        src.nch = rec.nch;
+        src.qc = rec.qc;
+        src.LP = LP;
+        src.slots = slots_s[wave];
+        src.lane = lane;
+        const uint32_t first_bucket = uint32_t(uni(level_buckets[l]));
+        auto groups = [&]<int NST>() __attribute__((always_inline)) {
+          for (int g = 0; g < src.nch; g += kRecordGroup) {
+            src.group(g, first_bucket, tile, tl.ntx, ty, bk.shift);
+            mfma_tile_kblocks<T, NB, NST>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
+          }
+        };
+        if (t.nst == 1)  // wave-uniform: a 4 x 4 tile runs one sub-tile's MFMAs
+          groups.template operator()<1>();
+        else
+          groups.template operator()<4>();
+      } else {
+        EntrySource<T, TL, SOFTMAX> src;
+        src.ent = entries + int64_t(bh) * bg.region;
+        src.cr = tile_candidates(buckets + int64_t(bh) * 4 * ntiles, tl, tile, tx, ty, uint32_t(l * p.P));
+        src.ncand = src.cr.ncand;
+        src.loc = p.loc + unit0 * LP * 2 * int64_t(sizeof(TL));
+        src.attn = p.attn + unit0 * LP * ES;
+        src.loc_q = uint32_t(p.H * LP * 2) * uint32_t(sizeof(TL));
+        src.attn_q = uint32_t(p.H * LP * ES);
+        src.div_lp = bg.div_lp;
+        src.LP = LP;
+        src.H = p.H;
+        src.stats = SOFTMAX && stats_ok ? (p.stats ? reinterpret_cast<const SoftStat<float>*>(p.stats)
+                                                   : softmax_stats<float>(buckets, p, 4 * ntiles)) + unit0
+                                        : nullptr;
+        src.lane = lane;
+        if (t.nst == 1)  // wave-uniform: a 4 x 4 tile runs one sub-tile's MFMAs
+          mfma_tile_kblocks<T, NB, 1>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
+        else
+          mfma_tile_kblocks<T, NB, 4>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
+      }
 
       T* gv = reinterpret_cast<T*>(p.grad_value);
       if (per_wave) {
@@ -3493,9 +3908,10 @@ int make_backward_plan(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, in
   return MSDA_OK;
 }
 
+// Lets a kernel take `bytes` of dynamic LDS (beside `fixed` of its own).
 template <typename Kernel>
-hipError_t allow_lds(Kernel k, size_t bytes) {
-  if (bytes <= 64 * 1024) return hipSuccess;
+hipError_t allow_lds(Kernel k, size_t bytes, size_t fixed = 0) {
+  if (bytes + fixed <= 64 * 1024) return hipSuccess;
   return hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                              int(bytes));
 }
@@ -3536,25 +3952,83 @@ hipError_t launch_owner_cvr(const BackwardPlan& plan, const Problem& p, const in
   return hipErrorInvalidValue;
 }
 
-template <typename T, typename TL, bool SM>
+template <typename T, typename TL, bool SM, bool RECORDS>
 hipError_t launch_owner_mfma(const BackwardPlan& plan, const Problem& p, const int* buckets,
-                             const uint32_t* entries, int accumulate, hipStream_t st) {
+                             const uint32_t* entries, const Records& rec, int accumulate, hipStream_t st) {
   if constexpr (std::is_same_v<T, bf16_t> || std::is_same_v<T, f16_t> || std::is_same_v<T, float>) {
     auto go = [&](auto k) -> hipError_t {
       const hipError_t e = allow_lds(k, plan.mfma_lds);
       if (e != hipSuccess) return e;
       hipLaunchKernelGGL(k, dim3(unsigned(plan.mfma_blocks)), dim3(kWave * kMfmaWaves), plan.mfma_lds, st, p,
-                         plan.bg, const_cast<int*>(buckets), entries, accumulate, plan.mfma_table);
+                         plan.bg, const_cast<int*>(buckets), entries, rec, accumulate, plan.mfma_table);
       return hipGetLastError();
     };
     switch (plan.mfma_nb) {
-      case 1: return go(msda_grad_value_mfma_kernel<T, TL, 1, SM>);
-      case 2: return go(msda_grad_value_mfma_kernel<T, TL, 2, SM>);
-      case 3: return go(msda_grad_value_mfma_kernel<T, TL, 3, SM>);
-      case 4: return go(msda_grad_value_mfma_kernel<T, TL, 4, SM>);
+      case 1: return go(msda_grad_value_mfma_kernel<T, TL, 1, SM, RECORDS>);
+      case 2: return go(msda_grad_value_mfma_kernel<T, TL, 2, SM, RECORDS>);
+      case 3: return go(msda_grad_value_mfma_kernel<T, TL, 3, SM, RECORDS>);
+      case 4: return go(msda_grad_value_mfma_kernel<T, TL, 4, SM, RECORDS>);
     }
   }
   return hipErrorInvalidValue;
+}
+
+// The record sort's chunks: RecordPlan::threads threads of `groups` groups of four
+// samples each. ok: the call takes it.
+struct RecordPlan {
+  bool ok;
+  int threads, groups, qc, nch;
+};
+
+// Chunks for a (b, h) of Q * LP samples whose bucket offsets (16 bits each) have
+// offs_cap entries of memory: the smallest of the workgroup sizes with which a tile's
+// ranges of every chunk still fit the lanes of one wave (kRecordGroup chunks), so that
+// small calls get many short workgroups; 16,384 samples (what 16-bit query and bucket
+// numbers and the LDS staging of a 1,024-thread workgroup allow) when none does, the
+// owners then taking the chunks in groups.
+RecordPlan make_record_plan(int64_t B, int64_t S, int64_t H, int64_t Q, int64_t L, int64_t P, bool small_tiles,
+                            int64_t offs_cap) {
+  static constexpr int kSizes[][2] = {{256, 1}, {512, 1}, {1024, 1}, {512, 4}, {1024, 4}};
+  RecordPlan r = {};
+  const int64_t LP = L * P;
+  // Tiles of levels of aspect ratio at most 16 that do not overlap (for others the kernels
+  // may take coarser buckets): h w / 64 + (h + w) / 8 + 1 per level, h + w <= 4.25
+  // sqrt(h w), and sum_l sqrt(h_l w_l) <= sqrt(L S); a level that takes 4 x 4 tiles has
+  // fewer than four times kSmallTileTasks / (B H).
+  const int64_t small =
+      small_tiles ? L * std::min<int64_t>(4 * (kSmallTileTasks / std::max<int64_t>(1, B * H) + 1), S / 16 + 1) : 0;
+  const int64_t tiles = S / 64 + int64_t(ceil(4.25 / 8 * sqrt(double(L) * double(S)))) + L + small;
+  for (const auto& size : kSizes) {
+    const int64_t n = int64_t(size[0]) * 4 * size[1];
+    const int64_t qc = n / LP;
+    if (qc < 1) continue;
+    const int64_t nch = (Q + qc - 1) / qc;
+    const bool last = n == 16384;
+    if ((nch > kRecordGroup && !last) || B * H * nch * (4 * tiles + 1) > offs_cap) continue;
+    if (xcd_group_grid(H, B * nch) >= 2147483647) continue;
+    r.ok = true;
+    r.threads = size[0];
+    r.groups = size[1];
+    r.qc = int(qc);
+    r.nch = int(nch);
+    break;
+  }
+  return r;
+}
+
+template <typename T, typename TL, bool SM>
+hipError_t launch_record_sort(const BackwardPlan& plan, const RecordPlan& rp, const Problem& p, const Records& rec,
+                              hipStream_t st) {
+  const size_t n = size_t(rp.threads) * 4 * rp.groups;
+  const size_t lds = n * std::max(2 * sizeof(TL), sizeof(RecordWeight<T, SM>) + 2);
+  auto go = [&](auto k) -> hipError_t {
+    const hipError_t e = allow_lds(k, lds, kRecordStaticLds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k, dim3(unsigned(xcd_group_grid(p.H, int64_t(p.B) * rec.nch))), dim3(unsigned(rp.threads)), lds,
+                       st, p, plan.bg, rec);
+    return hipGetLastError();
+  };
+  return rp.groups == 1 ? go(msda_record_sort_kernel<T, TL, SM, 1>) : go(msda_record_sort_kernel<T, TL, SM, 4>);
 }
 
 // The count, scan and place passes with SPT samples per bucketing thread.
@@ -3954,13 +4428,14 @@ static int backward_call(const void* value, int value_dtype, const void* spatial
   // A workspace of the full size gives the softmax statistics a region of their own.
   const bool ws_stats = use_ws && softmax && workspace_bytes >= wl.total;
   void* counters = use_ws ? static_cast<char*>(workspace) + wl.counters_off : grad_attention_weights;
+  const int paths = g_path_override.load(std::memory_order_relaxed);
   BackwardPlan plan;
   size_t lds_limit;
   int cus;
   device_info(&lds_limit, &cus);
   rc = make_backward_plan(value_dtype, batch, spatial, heads, channels, queries, levels, points,
                           loc_dtype, vec, 4, counters, lds_limit, cus, &plan, accumulate,
-                          g_path_override.load(std::memory_order_relaxed),
+                          paths,
                           !use_ws ? -1 : ws_stats ? wl.counters_bytes : workspace_bytes - wl.counters_off);
   if (rc != MSDA_OK) return rc;
   Problem p = make_problem(value, spatial_shapes, level_start_index, index_dtype,
@@ -3987,12 +4462,40 @@ static int backward_call(const void* value, int value_dtype, const void* spatial
   // workspace.
   int* buckets = static_cast<int*>(counters);
   uint32_t* entries = use_ws ? static_cast<uint32_t*>(workspace) : static_cast<uint32_t*>(grad_sampling_locations);
+  // The record sort, where it applies: four-sample groups with wide aligned accesses on
+  // both sides, its streams in the location and weight gradients (which grad_sample
+  // overwrites last) and the workspace's index region, its bucket offsets and work
+  // queue in the counters region. Records of 16-bit softmax weights hold them in
+  // float: those take the index region and the query numbers grad_attention_weights.
+  Records rec = {};
+  RecordPlan rp = {};
+  if (use_ws && plan.mfma && !plan.mfma_fallback && !atomic_gv && levels <= kRecordLevels && points % 4 == 0 &&
+      levels * points <= (softmax ? kRecordSoftmaxSamples : kRecordSamples) && spatial < kRecordPositions &&
+      aligned(sampling_locations, 16) && aligned(attention_weights, 4 * es) && aligned(grad_sampling_locations, 16) &&
+      aligned(grad_attention_weights, 4 * es) && !(paths & MSDA_PATH_ATOMIC_SORT)) {
+    const int64_t queue_bytes = int64_t(kXcds) * kQueueLine * 4;
+    const int64_t cap = (workspace_bytes - wl.counters_off - queue_bytes) / 2;
+    rp = make_record_plan(batch, spatial, heads, queries, levels, points, plan.bg.small_tiles, cap);
+    if (rp.ok) {
+      const bool wide = softmax && es == 2;  // 4-byte weights of 16-bit logits
+      rec.loc = static_cast<char*>(grad_sampling_locations);
+      rec.w = static_cast<char*>(wide ? workspace : grad_attention_weights);
+      rec.q = static_cast<uint16_t*>(wide ? grad_attention_weights : workspace);
+      rec.queue = static_cast<int*>(counters);
+      rec.offs = reinterpret_cast<uint16_t*>(static_cast<char*>(counters) + queue_bytes);
+      rec.offs_cap = cap;
+      rec.qc = rp.qc;
+      rec.nch = rp.nch;
+      plan.bg.div_gpq = make_fastdiv(uint32_t(levels * points / 4));
+      plan.bg.div_gpl = make_fastdiv(uint32_t(points / 4));
+    }
+  }
   // grad_sample beside the sort: it needs neither the sort nor grad_value, and with
   // the scratch in the workspace it writes nothing the sort uses. Only where it adds
   // nothing into grad_value (the matrix-core owners take every level, overlapping ones
   // included); it joins the caller's stream before the grad_value kernel.
   SideStream* side = nullptr;
-  if (fork && use_ws && p.sort_overlap && sample_count >= kSideStreamSamples && !g_phase_events_on) {
+  if (fork && use_ws && !rp.ok && p.sort_overlap && sample_count >= kSideStreamSamples && !g_phase_events_on) {
     side = side_stream();
     if (side == nullptr) return fail(MSDA_ERR_HIP, "msda_backward_workspace: no side stream: %s", hipGetErrorString(hipGetLastError()));
     // grad_sample, which forms each unit's softmax anyway, leaves the statistics for
@@ -4012,6 +4515,20 @@ static int backward_call(const void* value, int value_dtype, const void* spatial
         }
         record_phase(0, st);
         // The atomic scatter needs neither the sort nor the owners.
+        if constexpr (!std::is_same_v<T, double>) {
+          if (rp.ok) {
+            e = softmax ? launch_record_sort<T, TL, true>(plan, rp, p, rec, st)
+                        : launch_record_sort<T, TL, false>(plan, rp, p, rec, st);
+            record_phase(1, st);
+            if (e == hipSuccess)
+              e = softmax ? launch_owner_mfma<T, TL, true, true>(plan, p, nullptr, nullptr, rec, int(accumulate), st)
+                          : launch_owner_mfma<T, TL, false, true>(plan, p, nullptr, nullptr, rec, int(accumulate), st);
+            record_phase(2, st);
+            if (e == hipSuccess) e = launch_grad_sample<T, TL, CV>(plan, p, softmax, st);
+            record_phase(3, st);
+            return e;
+          }
+        }
         if (plan.bucket && !atomic_gv) {
           e = launch_buckets<TL>(plan, p, buckets, entries, st);
           if (e != hipSuccess) return e;
@@ -4040,8 +4557,8 @@ static int backward_call(const void* value, int value_dtype, const void* spatial
           if (e != hipSuccess) return e;
         }
         if (plan.mfma && !atomic_gv)
-          e = softmax ? launch_owner_mfma<T, TL, true>(plan, p, buckets, entries, int(accumulate), st)
-                      : launch_owner_mfma<T, TL, false>(plan, p, buckets, entries, int(accumulate), st);
+          e = softmax ? launch_owner_mfma<T, TL, true, false>(plan, p, buckets, entries, rec, int(accumulate), st)
+                      : launch_owner_mfma<T, TL, false, false>(plan, p, buckets, entries, rec, int(accumulate), st);
         if (e == hipSuccess && side && !p.stats) e = hipStreamWaitEvent(st, side->join, 0);
         if (e == hipSuccess && !atomic_gv && (!plan.mfma || plan.mfma_fallback)) {
           const int after_mfma = plan.mfma ? 1 : 0;

@@ -1,0 +1,61 @@
+"""The record sort and the owners over its streams (the workspace backward of calls
+with P a multiple of 4), against the float64 oracle and against the counting sort's
+path, at the sizes where they can go wrong: chunks that are exactly full, one sample
+short or a single query; more chunks than one wave holds ranges of; more buckets than
+the LDS counters; tables whose bucket offsets need coarse buckets; tile and level
+edges; heads of 16 to 64 channels; levels long and short enough for split and for
+per-wave tasks.
+
+Tolerances are the parity suite's: float32 1e-4 (grad_value's products of split 16-bit
+parts have relative error at most 3 * 2^-16 = 4.6e-5 each), 16-bit 2e-2 of the largest
+element (two roundings to bfloat16 are 2 * 2^-9 = 4e-3 of an element).
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from deformops_amd.backends.hip import _lib
+from tests.test_hip_msda import BWD_TOL, check_against_oracle, rel_err, run_hip
+from tests.workloads import make_workload
+
+pytestmark = pytest.mark.gpu
+
+F32, BF16, F16 = torch.float32, torch.bfloat16, torch.float16
+
+#: levels, batch, queries, heads, channels, points
+SHAPES = {
+    "one-query": (((1, 1),), 1, 1, 1, 16, 4),
+    "chunk-full": (((16, 16),), 1, 256, 2, 32, 4),
+    "chunk-and-one": (((16, 16),), 1, 257, 2, 32, 4),
+    "many-chunks": (((33, 31),), 1, 90001, 1, 16, 4),
+    "many-buckets": (((400, 400), (9, 9)), 1, 3000, 1, 16, 4),
+    "line": (((1, 20000),), 1, 20000, 1, 16, 4),
+    "lines": (((3, 7000), (9000, 1)), 1, 9000, 1, 16, 4),
+    "tile-edges": (((7, 9), (8, 8), (9, 17), (1, 1), (24, 16)), 2, 1003, 3, 48, 4),
+    "wide-heads": (((19, 25), (10, 13)), 1, 4001, 2, 64, 8),
+    "decoder": (((100, 134), (50, 67), (25, 34), (13, 17)), 2, 301, 4, 32, 4),
+    "coarse-and-fine": (((64, 64), (4, 4)), 2, 5000, 4, 32, 4),
+}
+DTYPES = [(F32, F32), (BF16, BF16), (F16, F16), (BF16, F32), (F16, F32)]
+
+
+@pytest.mark.parametrize("softmax", [False, True], ids=["linear", "softmax"])
+@pytest.mark.parametrize(("dtype", "loc_dtype"), DTYPES, ids=["f32", "bf16", "f16", "bf16-f32loc", "f16-f32loc"])
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_record_path_matches_the_oracle_and_the_counting_sort(device, shape, dtype, loc_dtype, softmax):
+    levels, B, Q, H, D, P = SHAPES[shape]
+    # A location gradient is a W (G01 - G00), of order W: at W = 20,000 it leaves f16's
+    # range (65,504), so the long levels take float32 locations there.
+    if max(max(side) for side in levels) > 4096 and loc_dtype is F16:
+        loc_dtype = F32
+    w = make_workload(2, batch=B, queries=Q, heads=H, channels=D, points=P, levels=levels, locations="uniform",
+                      seed=11).to(device, dtype, loc_dtype)
+    check_against_oracle(*w.operands(softmax=softmax), w.grad_output, softmax=softmax, dtype=dtype, label=shape)
+    got = run_hip(*w.operands(softmax=softmax), w.grad_output, softmax=softmax)
+    with _lib.path_override(_lib.PATH_ATOMIC_SORT):  # the counting sort
+        want = run_hip(*w.operands(softmax=softmax), w.grad_output, softmax=softmax)
+    assert rel_err(got[1], want[1].double().cpu()) <= BWD_TOL[dtype]
+    for g, r in zip(got[2:], want[2:]):  # the same kernel on the same inputs
+        torch.testing.assert_close(g, r, rtol=0, atol=0)
