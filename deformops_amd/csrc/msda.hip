@@ -2593,7 +2593,7 @@ template <typename T, typename TL, bool SOFTMAX> struct RecordSource {
   uint32_t pre, n;      // this lane's range: candidates before it, and in it
   uint32_t delta;       // record of its candidate j: j + delta
   uint32_t ncand;
-  int* slots;           // kWave ints of the wave's LDS
+  unsigned char* slots;  // kWave bytes of the wave's LDS
   int lane;
 
   struct Ref {
@@ -2644,7 +2644,7 @@ template <typename T, typename TL, bool SOFTMAX> struct RecordSource {
     wave_lds_order();
     slots[lane] = 0;
     wave_lds_order();
-    if (n > 0 && pre > first && rel < uint32_t(kWave)) slots[rel] = lane;
+    if (n > 0 && pre > first && rel < uint32_t(kWave)) slots[rel] = uint8_t(lane);
     wave_lds_order();
     const uint64_t before = __ballot(n > 0 && pre <= first);
     const int seed = before ? 63 - __builtin_clzll(before) : 0;
@@ -2900,9 +2900,9 @@ __device__ inline void mfma_tile_kblocks(const Source& src, const MfmaTile& t, c
 // owns these grad_value elements: one plain store each (a load-add-store with
 // `accumulate`).
 template <typename T, int NB>
-__device__ inline void mfma_store_subtile(const Problem& p, const Level& lv, const MfmaTile& t, int b, int h,
-                                          int st, const f32x4_v (&c)[NB], int g16, int i16, int accumulate,
-                                          T* gv, bool add = false) {
+__device__ inline void mfma_store_block(const Problem& p, const Level& lv, const MfmaTile& t, int b, int h, int st,
+                                        int nb, const f32x4_v& c, int g16, int i16, int accumulate, T* gv,
+                                        bool add = false) {
   constexpr int D = 16 * NB;
   // add (wave-uniform): overlapping levels. Tiles of two levels own the shared
   // positions, so each adds its fp32 sums with one atomic per element (float) or per
@@ -2917,31 +2917,36 @@ __device__ inline void mfma_store_subtile(const Problem& p, const Level& lv, con
     const int x = t.c0 + 4 * (st & 1) + r;
     const bool ok = yok && x < t.c1;
     const int64_t pos = int64_t(b) * p.S + lv.start + int64_t(y) * lv.w + x;
-    T* dst = gv + (pos * p.H + h) * D + i16;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      if (add) {
-        if constexpr (std::is_same_v<T, float>) {
-          if (ok) unsafeAtomicAdd(dst + 16 * nb, c[nb][r]);
-        } else {
-          const float pair = quad_perm<kQuadXor1>(c[nb][r]);
-          if (ok && (i16 & 1) == 0) {
-            if constexpr (std::is_same_v<T, bf16_t>) {
-              const bf16x2_v v2 = {static_cast<__bf16>(c[nb][r]), static_cast<__bf16>(pair)};
-              __builtin_amdgcn_global_atomic_fadd_v2bf16(reinterpret_cast<bf16x2_v*>(dst + 16 * nb), v2);
-            } else {
-              const f16x2_v v2 = {static_cast<_Float16>(c[nb][r]), static_cast<_Float16>(pair)};
-              __builtin_amdgcn_global_atomic_fadd_v2f16(reinterpret_cast<f16x2_v*>(dst + 16 * nb), v2);
-            }
+    T* dst = gv + (pos * p.H + h) * D + i16 + 16 * nb;
+    if (add) {
+      if constexpr (std::is_same_v<T, float>) {
+        if (ok) unsafeAtomicAdd(dst, c[r]);
+      } else {
+        const float pair = quad_perm<kQuadXor1>(c[r]);
+        if (ok && (i16 & 1) == 0) {
+          if constexpr (std::is_same_v<T, bf16_t>) {
+            const bf16x2_v v2 = {static_cast<__bf16>(c[r]), static_cast<__bf16>(pair)};
+            __builtin_amdgcn_global_atomic_fadd_v2bf16(reinterpret_cast<bf16x2_v*>(dst), v2);
+          } else {
+            const f16x2_v v2 = {static_cast<_Float16>(c[r]), static_cast<_Float16>(pair)};
+            __builtin_amdgcn_global_atomic_fadd_v2f16(reinterpret_cast<f16x2_v*>(dst), v2);
           }
         }
-      } else if (ok) {
-        float v = c[nb][r];
-        if (accumulate) v += load_acc(dst + 16 * nb);
-        store_elem(dst + 16 * nb, v);
       }
+    } else if (ok) {
+      float v = c[r];
+      if (accumulate) v += load_acc(dst);
+      store_elem(dst, v);
     }
   }
+}
+template <typename T, int NB>
+__device__ inline void mfma_store_subtile(const Problem& p, const Level& lv, const MfmaTile& t, int b, int h,
+                                          int st, const f32x4_v (&c)[NB], int g16, int i16, int accumulate,
+                                          T* gv, bool add = false) {
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+    mfma_store_block<T, NB>(p, lv, t, b, h, st, nb, c[nb], g16, i16, accumulate, gv, add);
 }
 
 // Workgroups per CU the register budget of the matrix-core kernel allows (float
@@ -2990,19 +2995,15 @@ __device__ inline int region_first_tile(int r, int n, int extent, int ntiles, in
 // early takes the next task of its queue. A small LDS table of prefix counts per
 // (pair, level) maps a queue position to its task. When the table would not fit,
 // queue x holds the x-th eighth of each level's tasks (b, tile, h) in raster order.
-// RECORDS: the candidates come from the record streams; else from `buckets` and
-// `entries`.
-template <typename T, typename TL, int NB, bool SOFTMAX, bool RECORDS>
+template <typename T, typename TL, int NB, bool SOFTMAX>
 __global__ __launch_bounds__(kWave * kMfmaWaves, mfma_blocks_per_cu(NB, int(sizeof(T)))) void msda_grad_value_mfma_kernel(
     const Problem p, const BwdGeom bg, int* __restrict__ buckets,
-    const uint32_t* __restrict__ entries, const Records rec, const int accumulate, const int table_cap) {
+    const uint32_t* __restrict__ entries, const int accumulate, const int table_cap) {
   constexpr int D = 16 * NB;
   constexpr int ES = int(sizeof(T));
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int wave_sums[kMfmaWaves];
   __shared__ int grid_s[2];
-  __shared__ int slots_s[RECORDS ? kMfmaWaves : 1][kWave];
-  __shared__ int level_buckets[RECORDS ? kRecordLevels : 1];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const int LP = p.L * p.P;
 
@@ -3052,10 +3053,8 @@ __global__ __launch_bounds__(kWave * kMfmaWaves, mfma_blocks_per_cu(NB, int(size
       }
     }
   }
-  if (ntiles <= 0 || (!RECORDS && !queue_fits(p, bg, 4 * ntiles))) return;  // the VALU owner kernel runs instead
-  RecordBuckets bk{};
-  if constexpr (RECORDS) bk = record_buckets(p, rec, lt, ntiles, level_buckets);
-  const bool stats_ok = SOFTMAX && !RECORDS && (p.stats || softmax_stats_fit<float>(p, bg, 4 * ntiles, buckets));
+  if (ntiles <= 0 || !queue_fits(p, bg, 4 * ntiles)) return;  // the VALU owner kernel runs instead
+  const bool stats_ok = SOFTMAX && (p.stats || softmax_stats_fit<float>(p, bg, 4 * ntiles, buckets));
   if (tid == 0) {
     order_levels(p, levels, lt, order, rank_base);
     // R x R regions, R the power of two nearest the finest level's tile count, at most
@@ -3086,10 +3085,9 @@ __global__ __launch_bounds__(kWave * kMfmaWaves, mfma_blocks_per_cu(NB, int(size
   __syncthreads();
 
   const int xcd = int(blockIdx.x) % kXcds;
-  int* queue = (RECORDS ? rec.queue
-                        : reinterpret_cast<int*>((reinterpret_cast<uintptr_t>(buckets + int64_t(p.B) * p.H * 4 * ntiles) +
-                                                  4 * kQueueLine - 1) &
-                                                 ~uintptr_t(4 * kQueueLine - 1))) +
+  int* queue = reinterpret_cast<int*>(
+                   (reinterpret_cast<uintptr_t>(buckets + int64_t(p.B) * p.H * 4 * ntiles) + 4 * kQueueLine - 1) &
+                   ~uintptr_t(4 * kQueueLine - 1)) +
                xcd * kQueueLine;
   const int64_t per_tile = int64_t(p.B) * p.H;
   const int R = grid_s[0];  // regions per axis, a power of two; visited in Morton order
@@ -3244,51 +3242,25 @@ __global__ __launch_bounds__(kWave * kMfmaWaves, mfma_blocks_per_cu(NB, int(size
         for (int j = 0; j < NB; ++j) acc[st][j] = f32x4_v{0.f, 0.f, 0.f, 0.f};
       // All K-blocks (per-wave mode), or K-blocks wave, wave + 4, ...
       const int kb0 = per_wave ? 0 : wave, kbstep = per_wave ? 1 : kMfmaWaves;
-      if constexpr (RECORDS) {
-        RecordSource<T, TL, SOFTMAX> src;
-        src.row = uint32_t(bk.count + 1);
-        const int64_t first = int64_t(bh) * p.Q * LP;
-        src.loc = rec.loc + first * 2 * int64_t(sizeof(TL));
-        src.w = reinterpret_cast<const RecordWeight<T, SOFTMAX>*>(rec.w) + first;
-        src.q = rec.q + first;
-        src.offs = rec.offs + int64_t(bh) * rec.nch * src.row;
-        src.nch = rec.nch;
-        src.qc = rec.qc;
-        src.LP = LP;
-        src.slots = slots_s[wave];
-        src.lane = lane;
-        const uint32_t first_bucket = uint32_t(uni(level_buckets[l]));
-        auto groups = [&]<int NST>() __attribute__((always_inline)) {
-          for (int g = 0; g < src.nch; g += kRecordGroup) {
-            src.group(g, first_bucket, tile, tl.ntx, ty, bk.shift);
-            mfma_tile_kblocks<T, NB, NST>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
-          }
-        };
-        if (t.nst == 1)  // wave-uniform: a 4 x 4 tile runs one sub-tile's MFMAs
-          groups.template operator()<1>();
-        else
-          groups.template operator()<4>();
-      } else {
-        EntrySource<T, TL, SOFTMAX> src;
-        src.ent = entries + int64_t(bh) * bg.region;
-        src.cr = tile_candidates(buckets + int64_t(bh) * 4 * ntiles, tl, tile, tx, ty, uint32_t(l * p.P));
-        src.ncand = src.cr.ncand;
-        src.loc = p.loc + unit0 * LP * 2 * int64_t(sizeof(TL));
-        src.attn = p.attn + unit0 * LP * ES;
-        src.loc_q = uint32_t(p.H * LP * 2) * uint32_t(sizeof(TL));
-        src.attn_q = uint32_t(p.H * LP * ES);
-        src.div_lp = bg.div_lp;
-        src.LP = LP;
-        src.H = p.H;
-        src.stats = SOFTMAX && stats_ok ? (p.stats ? reinterpret_cast<const SoftStat<float>*>(p.stats)
-                                                   : softmax_stats<float>(buckets, p, 4 * ntiles)) + unit0
-                                        : nullptr;
-        src.lane = lane;
-        if (t.nst == 1)  // wave-uniform: a 4 x 4 tile runs one sub-tile's MFMAs
-          mfma_tile_kblocks<T, NB, 1>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
-        else
-          mfma_tile_kblocks<T, NB, 4>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
-      }
+      EntrySource<T, TL, SOFTMAX> src;
+      src.ent = entries + int64_t(bh) * bg.region;
+      src.cr = tile_candidates(buckets + int64_t(bh) * 4 * ntiles, tl, tile, tx, ty, uint32_t(l * p.P));
+      src.ncand = src.cr.ncand;
+      src.loc = p.loc + unit0 * LP * 2 * int64_t(sizeof(TL));
+      src.attn = p.attn + unit0 * LP * ES;
+      src.loc_q = uint32_t(p.H * LP * 2) * uint32_t(sizeof(TL));
+      src.attn_q = uint32_t(p.H * LP * ES);
+      src.div_lp = bg.div_lp;
+      src.LP = LP;
+      src.H = p.H;
+      src.stats = SOFTMAX && stats_ok ? (p.stats ? reinterpret_cast<const SoftStat<float>*>(p.stats)
+                                                 : softmax_stats<float>(buckets, p, 4 * ntiles)) + unit0
+                                      : nullptr;
+      src.lane = lane;
+      if (t.nst == 1)  // wave-uniform: a 4 x 4 tile runs one sub-tile's MFMAs
+        mfma_tile_kblocks<T, NB, 1>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
+      else
+        mfma_tile_kblocks<T, NB, 4>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
 
       T* gv = reinterpret_cast<T*>(p.grad_value);
       if (per_wave) {
@@ -3323,6 +3295,249 @@ __global__ __launch_bounds__(kWave * kMfmaWaves, mfma_blocks_per_cu(NB, int(size
       mfma_zero_tiles(wt, lane);
     }
     __syncthreads();  // every wave is done with the chunk before the next one is published
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The owners over the record streams.
+//
+// One persistent workgroup per CU, of as many waves as its LDS and registers hold, and
+// per XCD two lists of (tile, image, head) tasks, levels of the heaviest tiles first.
+// The workgroups of an XCD first share its split tasks: all waves of a workgroup take
+// every W-th K-block of one task and the partial sums meet in LDS. Then every wave by
+// itself takes whole tasks, with no barrier between them. Heaviest first, and split
+// where a task alone would outlast the rest, because the call waits for its last task:
+// in queue order of image regions, tasks of 80 us that started late kept a 150 us
+// kernel's waves idle for a fifth of it (B = 4, Q = 21,504 bf16). The order no longer
+// follows image regions: with the records read in order, only the grad_out rows are
+// gathered, and reading them from one hot line instead changes the time by 1 %.
+constexpr int record_owner_waves(int nb, int es) {
+  return es == 4 ? (nb == 1 ? 12 : nb == 2 ? 8 : 4) : (nb <= 2 ? 12 : 8);
+}
+
+// When a level's tasks are split over a workgroup (K-blocks expected per task).
+constexpr float kSplitKBlocks = 3.f;  // and at least twice a wave's average work
+constexpr int kSplitRounds = 6;       // or this many K-blocks for every wave
+constexpr float kShortKBlocks = 2.f;  // a short task has at most this many, expected
+
+template <typename T, typename TL, int NB, bool SOFTMAX>
+__global__ __launch_bounds__(kWave * record_owner_waves(NB, int(sizeof(T))),
+                             (record_owner_waves(NB, int(sizeof(T))) + 3) / 4) void
+msda_record_owner_kernel(const Problem p, const BwdGeom bg, const Records rec, const int accumulate) {
+  constexpr int D = 16 * NB;
+  constexpr int ES = int(sizeof(T));
+  constexpr int kWaves = record_owner_waves(NB, ES);
+  constexpr bool kSplit = sizeof(T) == 4;
+  constexpr size_t kRowsBytes = size_t(kMfmaK) * size_t(mfma_row_bytes(NB)) * (kSplit ? 2 : 1);
+  constexpr size_t kWaveBytes = std::max(kRowsBytes + size_t(kMfmaTileBytes), size_t(4 * NB * kWave * 16));
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ Level levels[kRecordLevels];
+  __shared__ LevelTiles lt[kRecordLevels];
+  __shared__ int level_buckets[kRecordLevels];
+  __shared__ int64_t total;
+  __shared__ float work_s[kRecordLevels];        // expected K-blocks per task
+  __shared__ int order_s[kRecordLevels];         // levels, heaviest tasks first
+  __shared__ int split_end_s[kRecordLevels], wave_end_s[kRecordLevels];  // list positions after each ordered level
+  __shared__ int next_s[2];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uni(tid / kWave);
+  const int LP = p.L * p.P;
+  unsigned char* gst = smem + size_t(wave) * kWaveBytes;  // grad_out rows (hi, then lo)
+  unsigned char* wt = gst + kRowsBytes;                   // eight weight tiles (hi, then lo)
+
+  bool overlap;
+  const int64_t ntiles = load_tiles(p, bg, levels, lt, &total, &overlap);
+  // Overlapping levels: the sort zeroed grad_value, and the owners add.
+  const bool add = overlap;
+  if (!accumulate && !add) {
+    // grad_value at positions no valid level covers is zero (the tiles own the others).
+    const int64_t n = int64_t(p.B) * p.S;
+    for (int64_t idx = int64_t(blockIdx.x) * blockDim.x + tid; idx < n; idx += int64_t(gridDim.x) * blockDim.x) {
+      const int pos = int(idx % p.S);
+      bool covered = false;
+      for (int l = 0; l < p.L && !covered; ++l) {
+        const Level lv = levels[l];
+        covered = lv.ok && pos >= lv.start && int64_t(pos) < int64_t(lv.start) + int64_t(lv.h) * lv.w;
+      }
+      if (!covered) {
+        T* dst = reinterpret_cast<T*>(p.grad_value) + idx * p.H * D;
+        for (int i = 0; i < p.H * D; ++i) store_elem(dst + i, 0.f);
+      }
+    }
+  }
+  if (ntiles <= 0) return;
+  const RecordBuckets bk = record_buckets(p, rec, lt, ntiles, level_buckets);
+
+  // The lists. A level's tasks are split over the workgroup when one is longer than
+  // twice what a wave gets on average, or so long that the merge does not matter.
+  const int xcd = int(blockIdx.x) % kXcds, slot = int(blockIdx.x) / kXcds;
+  const int slots = int(gridDim.x) / kXcds;
+  const int per_tile = p.B * p.H;
+  if (tid < p.L) {
+    const LevelTiles t = lt[tid];
+    const int n = t.ntx * t.nty;
+    const float side = float(1 << t.lw), straddle = (1.f + 1.f / side) * (1.f + 1.f / side);
+    work_s[tid] = n > 0 ? float(p.Q) * float(p.P) * straddle / (float(kMfmaK) * float(n)) : 0.f;
+  }
+  __syncthreads();
+  if (tid < p.L) {
+    int rank = 0;
+    float all = 0.f;
+    for (int l = 0; l < p.L; ++l) {
+      const float w = work_s[l];
+      rank += w > work_s[tid] || (w == work_s[tid] && l < tid) ? 1 : 0;
+      all += w * float(lt[l].ntx * lt[l].nty);
+    }
+    const float average = all * float(per_tile) / (float(gridDim.x) * float(kWaves));
+    const float w = work_s[tid];
+    const bool split = w >= kSplitKBlocks && w >= 2.f * average || w >= float(kSplitRounds * kWaves);
+    const int64_t n = int64_t(lt[tid].ntx * lt[tid].nty) * per_tile;
+    const int mine = int((xcd + 1) * n / kXcds - xcd * n / kXcds);
+    order_s[rank] = tid;
+    split_end_s[rank] = split ? mine : 0;
+    wave_end_s[rank] = split ? 0 : mine;
+  }
+  __syncthreads();
+  int nsplit = 0, nwave = 0, short_from = 0;
+  for (int i = 0; i < p.L; ++i) {
+    nsplit += split_end_s[i];
+    nwave += wave_end_s[i];
+    if (work_s[order_s[i]] > kShortKBlocks) short_from = nwave;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int a = 0, b = 0;
+    for (int i = 0; i < p.L; ++i) {
+      split_end_s[i] = a += split_end_s[i];
+      wave_end_s[i] = b += wave_end_s[i];
+    }
+  }
+  __syncthreads();
+  nsplit = uni(nsplit);
+  nwave = uni(nwave);
+  int* split_queue = rec.queue + xcd * kQueueLine;
+  int* wave_queue = split_queue + 1;
+  const int g16 = lane >> 4, i16 = lane & 15;
+  T* gv = reinterpret_cast<T*>(p.grad_value);
+  mfma_zero_tiles(wt, lane);
+
+  // One task: its K-blocks kb0, kb0 + kbstep, ... into acc.
+  struct Task {
+    MfmaTile t;
+    Level lv;
+    int b, h;
+  };
+  // The task at position k of a list, and its candidate source.
+  RecordSource<T, TL, SOFTMAX> src;
+  src.row = uint32_t(bk.count + 1);
+  src.nch = rec.nch;
+  src.qc = rec.qc;
+  src.LP = LP;
+  src.slots = wt + kMfmaSpare;
+  src.lane = lane;
+  auto run = [&](int k, const int* ends, int kb0, int kbstep, f32x4_v (&acc)[4][NB], int& parts) __attribute__((always_inline)) -> Task {
+    int oi = 0;
+    while (oi + 1 < p.L && k >= ends[oi]) ++oi;
+    const int l = uni(order_s[oi]);
+    Level lv = levels[l];
+    lv = Level{uni(lv.h), uni(lv.w), uni(lv.start), uni(lv.ok)};
+    LevelTiles tl = lt[l];
+    tl = LevelTiles{uni(tl.lh), uni(tl.lw), uni(tl.ntx), uni(tl.nty), uni(tl.base)};
+    const int ntl = tl.ntx * tl.nty;
+    const int64_t n = int64_t(ntl) * per_tile;
+    const uint32_t task = uint32_t(xcd * n / kXcds) + uint32_t(k - (oi > 0 ? uni(ends[oi - 1]) : 0));
+    const uint32_t rest = task / uint32_t(p.H);
+    const int h = uni(int(task - rest * uint32_t(p.H))), b = uni(int(rest / uint32_t(ntl)));
+    const int tile = uni(int(rest - uint32_t(b) * uint32_t(ntl)));
+    const int ty = uni(tile / tl.ntx), tx = tile - ty * tl.ntx;
+    const int64_t bh = int64_t(b) * p.H + h;
+    Task r;
+    r.lv = lv;
+    r.b = b;
+    r.h = h;
+    MfmaTile& t = r.t;
+    t.gout = p.grad_out + (int64_t(b) * p.Q * p.H + h) * D * ES;
+    t.gout_q = uint32_t(p.H * D * ES);
+    t.r0 = ty << tl.lh;
+    t.c0 = tx << tl.lw;
+    t.r1 = min(t.r0 + (1 << tl.lh), lv.h);
+    t.c1 = min(t.c0 + (1 << tl.lw), lv.w);
+    t.nst = tl.lw < kMfmaSubLog2 ? 1 : 4;  // a 4 x 4 tile is sub-tile 0 alone
+    const int64_t first = bh * p.Q * LP;
+    src.loc = rec.loc + first * 2 * int64_t(sizeof(TL));
+    src.w = reinterpret_cast<const RecordWeight<T, SOFTMAX>*>(rec.w) + first;
+    src.q = rec.q + first;
+    src.offs = rec.offs + bh * rec.nch * src.row;
+    const uint32_t first_bucket = uint32_t(uni(level_buckets[l]));
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[st][j] = f32x4_v{0.f, 0.f, 0.f, 0.f};
+    parts = 0;
+    auto groups = [&]<int NST>() __attribute__((always_inline)) {
+      for (int g = 0; g < src.nch; g += kRecordGroup) {
+        src.group(g, first_bucket, tile, tl.ntx, ty, bk.shift);
+        parts = max(parts, int((src.ncand + kMfmaK - 1) / kMfmaK));
+        mfma_tile_kblocks<T, NB, NST>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
+      }
+    };
+    if (t.nst == 1)  // wave-uniform: a 4 x 4 tile runs one sub-tile's MFMAs
+      groups.template operator()<1>();
+    else
+      groups.template operator()<4>();
+    return r;
+  };
+
+  f32x4_v acc[4][NB];
+  for (int k = slot; k < nsplit;) {
+    if (tid == 0) next_s[0] = slots + atomicAdd(split_queue, 1);
+    int parts;
+    const Task r = run(k, split_end_s, wave, kWaves, acc, parts);
+    parts = min(parts, kWaves);  // waves that had K-blocks
+    u32x4_v* out = reinterpret_cast<u32x4_v*>(gst);
+    if (wave < parts)
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) out[(st * NB + nb) * kWave + lane] = __builtin_bit_cast(u32x4_v, acc[st][nb]);
+    __syncthreads();
+    // Sub-tile and channel block u of the sums: wave u % W.
+    for (int u = wave; u < 4 * NB; u += kWaves) {
+      f32x4_v sum = f32x4_v{0.f, 0.f, 0.f, 0.f};
+      for (int w = 0; w < parts; ++w)
+        sum += __builtin_bit_cast(f32x4_v, reinterpret_cast<const u32x4_v*>(smem + size_t(w) * kWaveBytes)[u * kWave + lane]);
+      if (u / NB < r.t.nst)
+        mfma_store_block<T, NB>(p, r.lv, r.t, r.b, r.h, u / NB, u % NB, sum, g16, i16, accumulate, gv, add);
+    }
+    k = next_s[0];
+    __syncthreads();  // the sums and the next task are read
+    if (wave < parts) mfma_zero_tiles(wt, lane);
+  }
+  // Waves that never had split tasks to wait for start on a task of their own each.
+  int k = nsplit == 0 ? slot * kWaves + wave : -1;
+  const int base = nsplit == 0 ? slots * kWaves : 0;
+  if (k < 0) {
+    int v = 0;
+    if (lane == 0) v = atomicAdd(wave_queue, 1);
+    k = uni(v);
+  }
+  while (k < nwave) {
+    // The next task is taken when this one is nearly done: a wave that took it at the
+    // start would hold back a long task that another could begin. Among short ones
+    // (`short_from` on) it is taken at the start, to hide the fetch.
+    int next = 0;
+    const bool early = k >= short_from;
+    if (early && lane == 0) next = atomicAdd(wave_queue, 1);
+    int parts;
+    const Task r = run(k, wave_end_s, 0, 1, acc, parts);
+    if (!early && lane == 0) next = atomicAdd(wave_queue, 1);
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+      if (st < r.t.nst) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          mfma_store_block<T, NB>(p, r.lv, r.t, r.b, r.h, st, nb, acc[st][nb], g16, i16, accumulate, gv, add);
+      }
+    k = base + uni(next);
   }
 }
 
@@ -3952,22 +4167,22 @@ hipError_t launch_owner_cvr(const BackwardPlan& plan, const Problem& p, const in
   return hipErrorInvalidValue;
 }
 
-template <typename T, typename TL, bool SM, bool RECORDS>
+template <typename T, typename TL, bool SM>
 hipError_t launch_owner_mfma(const BackwardPlan& plan, const Problem& p, const int* buckets,
-                             const uint32_t* entries, const Records& rec, int accumulate, hipStream_t st) {
+                             const uint32_t* entries, int accumulate, hipStream_t st) {
   if constexpr (std::is_same_v<T, bf16_t> || std::is_same_v<T, f16_t> || std::is_same_v<T, float>) {
     auto go = [&](auto k) -> hipError_t {
       const hipError_t e = allow_lds(k, plan.mfma_lds);
       if (e != hipSuccess) return e;
       hipLaunchKernelGGL(k, dim3(unsigned(plan.mfma_blocks)), dim3(kWave * kMfmaWaves), plan.mfma_lds, st, p,
-                         plan.bg, const_cast<int*>(buckets), entries, rec, accumulate, plan.mfma_table);
+                         plan.bg, const_cast<int*>(buckets), entries, accumulate, plan.mfma_table);
       return hipGetLastError();
     };
     switch (plan.mfma_nb) {
-      case 1: return go(msda_grad_value_mfma_kernel<T, TL, 1, SM, RECORDS>);
-      case 2: return go(msda_grad_value_mfma_kernel<T, TL, 2, SM, RECORDS>);
-      case 3: return go(msda_grad_value_mfma_kernel<T, TL, 3, SM, RECORDS>);
-      case 4: return go(msda_grad_value_mfma_kernel<T, TL, 4, SM, RECORDS>);
+      case 1: return go(msda_grad_value_mfma_kernel<T, TL, 1, SM>);
+      case 2: return go(msda_grad_value_mfma_kernel<T, TL, 2, SM>);
+      case 3: return go(msda_grad_value_mfma_kernel<T, TL, 3, SM>);
+      case 4: return go(msda_grad_value_mfma_kernel<T, TL, 4, SM>);
     }
   }
   return hipErrorInvalidValue;
@@ -4029,6 +4244,31 @@ hipError_t launch_record_sort(const BackwardPlan& plan, const RecordPlan& rp, co
     return hipGetLastError();
   };
   return rp.groups == 1 ? go(msda_record_sort_kernel<T, TL, SM, 1>) : go(msda_record_sort_kernel<T, TL, SM, 4>);
+}
+
+template <typename T, typename TL, bool SM>
+hipError_t launch_record_owner(const BackwardPlan& plan, const Problem& p, const Records& rec, int accumulate, int cus,
+                               hipStream_t st) {
+  if constexpr (!std::is_same_v<T, double>) {
+    auto go = [&]<int NB>() -> hipError_t {
+      auto k = msda_record_owner_kernel<T, TL, NB, SM>;
+      constexpr int kWaves = record_owner_waves(NB, int(sizeof(T)));
+      const size_t lds = size_t(kWaves) * mfma_wave_bytes(16 * NB, sizeof(T) == 4);
+      const hipError_t e = allow_lds(k, lds, kRecordStaticLds);
+      if (e != hipSuccess) return e;
+      // One workgroup per CU, a multiple of the XCDs.
+      const unsigned blocks = unsigned((cus + kXcds - 1) / kXcds * kXcds);
+      hipLaunchKernelGGL(k, dim3(blocks), dim3(kWave * kWaves), lds, st, p, plan.bg, rec, accumulate);
+      return hipGetLastError();
+    };
+    switch (plan.mfma_nb) {
+      case 1: return go.template operator()<1>();
+      case 2: return go.template operator()<2>();
+      case 3: return go.template operator()<3>();
+      case 4: return go.template operator()<4>();
+    }
+  }
+  return hipErrorInvalidValue;
 }
 
 // The count, scan and place passes with SPT samples per bucketing thread.
@@ -4521,8 +4761,8 @@ static int backward_call(const void* value, int value_dtype, const void* spatial
                         : launch_record_sort<T, TL, false>(plan, rp, p, rec, st);
             record_phase(1, st);
             if (e == hipSuccess)
-              e = softmax ? launch_owner_mfma<T, TL, true, true>(plan, p, nullptr, nullptr, rec, int(accumulate), st)
-                          : launch_owner_mfma<T, TL, false, true>(plan, p, nullptr, nullptr, rec, int(accumulate), st);
+              e = softmax ? launch_record_owner<T, TL, true>(plan, p, rec, int(accumulate), cus, st)
+                          : launch_record_owner<T, TL, false>(plan, p, rec, int(accumulate), cus, st);
             record_phase(2, st);
             if (e == hipSuccess) e = launch_grad_sample<T, TL, CV>(plan, p, softmax, st);
             record_phase(3, st);
@@ -4557,8 +4797,8 @@ static int backward_call(const void* value, int value_dtype, const void* spatial
           if (e != hipSuccess) return e;
         }
         if (plan.mfma && !atomic_gv)
-          e = softmax ? launch_owner_mfma<T, TL, true, false>(plan, p, buckets, entries, rec, int(accumulate), st)
-                      : launch_owner_mfma<T, TL, false, false>(plan, p, buckets, entries, rec, int(accumulate), st);
+          e = softmax ? launch_owner_mfma<T, TL, true>(plan, p, buckets, entries, int(accumulate), st)
+                      : launch_owner_mfma<T, TL, false>(plan, p, buckets, entries, int(accumulate), st);
         if (e == hipSuccess && side && !p.stats) e = hipStreamWaitEvent(st, side->join, 0);
         if (e == hipSuccess && !atomic_gv && (!plan.mfma || plan.mfma_fallback)) {
           const int after_mfma = plan.mfma ? 1 : 0;
