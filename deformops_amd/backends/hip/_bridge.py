@@ -30,7 +30,7 @@ from torch import Tensor
 
 from ...core.runtime import Method
 from ...registry import MSDAContext, resolve_msda_attn
-from . import _lib
+from . import _lib, _native
 
 __all__ = [
     "NAMESPACE",
@@ -243,37 +243,11 @@ forward_op, backward_op = _define("msda", softmax=False)
 forward_softmax_op, backward_softmax_op = _define("msda_softmax", softmax=True)
 
 
-class _EagerMSDA(torch.autograd.Function):
-    """The private operators' forward and backward for plain eager calls.
-
-    The same two library calls as the registered operators, without the custom-op
-    dispatch around each (argument defaults, redispatch, the autograd wrapper), which
-    costs more host time than a small call's kernels. Traced, compiled, exported and
-    fake calls use the registered operators.
-    """
-
-    @staticmethod
-    def forward(ctx, value, spatial_shapes, level_start_index, loc, attn, softmax):  # noqa: ANN001, ANN205, PLR0913
-        # The operands come normalized from `forward` below.
-        ctx.save_for_backward(value, spatial_shapes, level_start_index, loc, attn)
-        ctx.softmax = softmax
-        return _launch_forward(value, spatial_shapes, level_start_index, loc, attn, softmax=softmax)
-
-    @staticmethod
-    @torch.autograd.function.once_differentiable
-    def backward(ctx, grad_output):  # noqa: ANN001, ANN205
-        # The kernels' gradients carry no graph: a second derivative raises, as the
-        # reference's CUDA bridge does (cuda/_msda_bridge.py:232).
-        value, spatial_shapes, level_start_index, loc, attn = ctx.saved_tensors
-        grad_value, grad_loc, grad_attn = _launch_backward(
-            value, spatial_shapes, level_start_index, loc, attn, grad_output, softmax=ctx.softmax
-        )
-        return grad_value, None, None, grad_loc, grad_attn, None
-
-
 def _plain_eager(*tensors: Tensor) -> bool:
     """Real tensors, no compile / trace, no dispatch or function mode, no functorch wrapper."""
     if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack():  # noqa: SLF001
+        return False
+    if torch._C._get_tracing_state() is not None:  # noqa: SLF001
         return False
     if torch._C._is_torch_function_mode_enabled():  # noqa: SLF001
         return False
@@ -312,12 +286,16 @@ def forward(
         raise RuntimeError(msg)
     if num_points is None:
         num_points = int(sampling_locations.shape[4])
+    if _plain_eager(value, spatial_shapes, level_start_index, sampling_locations, attention_weights):
+        # The same two library calls as the registered operators, in one native autograd
+        # node (csrc/bridge.cpp). Traced, compiled, exported and fake calls use the
+        # operators.
+        _check_points(sampling_locations, num_points)
+        return _native.load().forward(value, spatial_shapes, level_start_index, sampling_locations,
+                                      attention_weights, softmax)
     operands = _normalized(value, spatial_shapes, level_start_index, sampling_locations, attention_weights)
     # The kernels take the operands in their own dtypes: no autocast inside.
     with torch.autocast("cuda", enabled=False) if torch.is_autocast_enabled("cuda") else contextlib.nullcontext():
-        if _plain_eager(*operands):
-            _check_points(operands[3], num_points)
-            return _EagerMSDA.apply(*operands, softmax)
         op = forward_softmax_op if softmax else forward_op
         return op(*operands, chunk_step, num_points, channels_per_thread, threads_per_block)
 

@@ -8,7 +8,7 @@ import torch
 
 from ...core.runtime import Method, resolve_method
 from ...registry import Backend, msda
-from . import _lib
+from . import _lib, _native
 from ._bridge import forward, supports_context
 
 
@@ -44,11 +44,19 @@ def msda_hip(
 
 
 def load(*, download: bool | None = None, compile: bool | str | None = None) -> str:  # noqa: A002
-    """Load libdeformops_amd.so and return its path."""
-    return str(_lib.load(download=download, compile=compile).path)
+    """Load libdeformops_amd.so and its native bridge; return the library's path."""
+    path = str(_lib.load(download=download, compile=compile).path)
+    _native.load()
+    return path
+
+
+def direct(*tensors: Any, softmax: bool) -> Any:
+    """A plain eager GPU call that needs no check the native bridge cannot make, or
+    ``None`` (see ``try_forward`` in csrc/bridge.cpp)."""
+    return _native.load().try_forward(*tensors, softmax)
 
 
 if torch.cuda.is_available() and torch.version.hip is not None:
-    msda.register(Backend.HIP, msda_hip, supports=supports_context, load=load)
+    msda.register(Backend.HIP, msda_hip, supports=supports_context, load=load, direct=direct)
 else:
     msda.mark_unavailable(Backend.HIP, "no ROCm GPU is available to this process")

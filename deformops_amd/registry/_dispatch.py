@@ -80,6 +80,7 @@ class _Entry:
     run: Callable[..., Any]
     supports: Callable[[Any], bool] | None = None
     load: Callable[..., Any] | None = None
+    direct: Callable[..., Any] | None = None
 
 
 #: Packages that hold each backend's adapter module (``<package>.<operator>``).
@@ -164,11 +165,14 @@ class Registry:
         *,
         supports: Callable[[Any], bool] | None = None,
         load: Callable[..., Any] | None = None,
+        direct: Callable[..., Any] | None = None,
     ) -> None:
         """File ``op_handle`` as ``backend``'s implementation, with an optional
-        ``supports(context)`` predicate and ``load(download=, compile=)`` hook."""
+        ``supports(context)`` predicate, ``load(download=, compile=)`` hook and
+        ``direct`` call (a route may try it in place of the checked call; it answers
+        ``None`` for a call it leaves to that)."""
         _require_backend(backend, allow_none=False)
-        self._entries[backend] = _Entry(op_handle, supports, load)
+        self._entries[backend] = _Entry(op_handle, supports, load, direct)
         self._absent.pop(backend, None)
         self._chosen.clear()
 
@@ -181,6 +185,11 @@ class Registry:
     def route_selected_calls(self, route: Callable[..., Any]) -> None:
         """Send ``backend=None`` calls through ``route`` (the public operator)."""
         self._route = route
+
+    def direct(self, backend: Backend) -> Callable[..., Any] | None:
+        """``backend``'s direct call, when its adapter is imported and has one."""
+        entry = self._entries.get(backend)
+        return None if entry is None else entry.direct
 
     def _import_adapters(self) -> None:
         if self._adapters_ready:

@@ -275,6 +275,14 @@ def _route_selected(*args: Any, method: str | Method | None = None, softmax: boo
                     **options: Any) -> Tensor:
     """A ``backend=None`` call: the public operator, or the same work directly when
     plain eager; backend options go to the selected backend."""
+    if not options and len(args) == 5 and not torch.compiler.is_compiling():  # noqa: PLR2004
+        # The host time of a small call is longer than its kernels: the native bridge
+        # makes the checks below itself where they pass, and leaves the rest to them.
+        direct = msda.direct(Backend.HIP)
+        if direct is not None:
+            out = direct(*args, softmax=resolve_method(method, softmax=softmax) is Method.SOFTMAX)
+            if out is not None:
+                return out
     if any(name in _BACKEND_OPTIONS for name in options):
         return msda.run_selected(*args, method=method, softmax=softmax, **options)
     tensors = _operands(args, options)
