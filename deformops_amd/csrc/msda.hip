@@ -396,21 +396,23 @@ template <typename A> struct alignas(16) Staged {
   A w[4];
 };
 
-__device__ inline void load_levels(const Problem& p, Level* levels) {
-  for (int i = threadIdx.x; i < p.L; i += blockDim.x) {
-    int64_t h, w, st;
-    if (p.index_i32) {
-      h = static_cast<const int32_t*>(p.shapes)[2 * i];
-      w = static_cast<const int32_t*>(p.shapes)[2 * i + 1];
-      st = static_cast<const int32_t*>(p.starts)[i];
-    } else {
-      h = static_cast<const int64_t*>(p.shapes)[2 * i];
-      w = static_cast<const int64_t*>(p.shapes)[2 * i + 1];
-      st = static_cast<const int64_t*>(p.starts)[i];
-    }
-    const bool ok = h > 0 && w > 0 && st >= 0 && h <= p.S && w <= p.S && st + h * w <= p.S;
-    levels[i] = ok ? Level{int(h), int(w), int(st), 1} : Level{1, 1, 0, 0};
+__device__ inline Level load_level(const Problem& p, int i) {
+  int64_t h, w, st;
+  if (p.index_i32) {
+    h = static_cast<const int32_t*>(p.shapes)[2 * i];
+    w = static_cast<const int32_t*>(p.shapes)[2 * i + 1];
+    st = static_cast<const int32_t*>(p.starts)[i];
+  } else {
+    h = static_cast<const int64_t*>(p.shapes)[2 * i];
+    w = static_cast<const int64_t*>(p.shapes)[2 * i + 1];
+    st = static_cast<const int64_t*>(p.starts)[i];
   }
+  const bool ok = h > 0 && w > 0 && st >= 0 && h <= p.S && w <= p.S && st + h * w <= p.S;
+  return ok ? Level{int(h), int(w), int(st), 1} : Level{1, 1, 0, 0};
+}
+
+__device__ inline void load_levels(const Problem& p, Level* levels) {
+  for (int i = threadIdx.x; i < p.L; i += blockDim.x) levels[i] = load_level(p, i);
 }
 
 // Whether this thread's levels (i = threadIdx.x, + blockDim.x, ...) share positions
@@ -1575,31 +1577,58 @@ template <typename T, bool SOFTMAX> using RecordWeight = std::conditional_t<SOFT
 // Bucket of a sample for the record sort: 4 * tile + position of its sub-bucket.
 __device__ inline int record_bucket(int key) { return (key & ~3) | ((key + 1) & 3); }
 
-// The buckets of a chunk: four per tile (shift < 0), or, where the offsets of those do
-// not fit their memory (levels far from square, or overlapping ones: the host knows
+// What the record kernels plan from the level table, in LDS: the levels and their tiles,
+// and the buckets of a chunk: four per tile (shift < 0), or, where the offsets of those
+// do not fit their memory (levels far from square, or overlapping ones: the host knows
 // only S and L), one per 2^shift consecutive tiles of a level. A tile then reads whole
 // buckets and ignores the samples that do not reach it.
-struct RecordBuckets {
-  int shift, count;
+struct RecordLevels {
+  Level level[kRecordLevels];
+  LevelTiles tiles[kRecordLevels];
+  int first[kRecordLevels];  // first bucket of the level
+  int ntiles, shift, buckets;
+  int overlap;  // two valid levels share positions of S
 };
-// Whole workgroup; `first` (shared) gets every level's first bucket. One barrier.
-__device__ inline RecordBuckets record_buckets(const Problem& p, const Records& r, const LevelTiles* lt,
-                                               int64_t ntiles, int* first) {
+
+// Lane l of the first wave plans level l, with no barrier between the steps (the caller
+// needs one before it reads the plan). Fewer than 2^20 positions and at most 16 levels:
+// 32-bit counts.
+__device__ inline RecordLevels& plan_records(const Problem& p, const BwdGeom& bg, const Records& r, RecordLevels& out) {
+  const int l = int(threadIdx.x);
+  const bool mine = l < p.L;
+  const Level lv = mine ? load_level(p, l) : Level{1, 1, 0, 0};
+  LevelTiles t = level_tiles(p, bg, lv);
+  const int nt = t.ntx * t.nty;
+  const int a0 = lv.start, a1 = lv.start + lv.h * lv.w;
+  bool any = false;
+  for (int j = 0; j < p.L; ++j) {
+    const int b0 = __builtin_amdgcn_readlane(a0, j), b1 = __builtin_amdgcn_readlane(a1, j);
+    any = any || (j != l && lv.ok && __builtin_amdgcn_readlane(lv.ok, j) && a0 < b1 && b0 < a1);
+  }
+  const int inc = wave_inclusive_scan(nt);
+  t.base = inc - nt;
+  const int ntiles = __builtin_amdgcn_readlane(inc, kWave - 1);
   const int64_t rows = int64_t(p.B) * p.H * r.nch;
-  RecordBuckets b{-1, int(4 * ntiles)};
-  if (rows * (4 * ntiles + 1) > r.offs_cap) {
-    b.shift = 0;
-    while (rows * ((ntiles >> b.shift) + p.L + 1) > r.offs_cap && b.shift < 30) ++b.shift;
+  int shift = -1;
+  if (rows * (4 * int64_t(ntiles) + 1) > r.offs_cap) {
+    shift = 0;
+    while (rows * ((ntiles >> shift) + p.L + 1) > r.offs_cap && shift < 30) ++shift;
   }
-  int at = 0;
-  for (int l = 0; l < p.L; ++l) {
-    const int nt = lt[l].ntx * lt[l].nty;
-    if (threadIdx.x == 0) first[l] = at;
-    at += b.shift < 0 ? 4 * nt : (nt + (1 << b.shift) - 1) >> b.shift;
+  const int nb = shift < 0 ? 4 * nt : (nt + (1 << shift) - 1) >> shift;
+  const int binc = wave_inclusive_scan(nb);
+  if (mine) {
+    out.level[l] = lv;
+    out.tiles[l] = t;
+    out.first[l] = binc - nb;
   }
-  b.count = at;
-  __syncthreads();
-  return b;
+  const bool overlap = __any(any);
+  if (l == 0) {
+    out.ntiles = ntiles;
+    out.shift = shift;
+    out.buckets = __builtin_amdgcn_readlane(binc, kWave - 1);
+    out.overlap = overlap;
+  }
+  return out;
 }
 
 // One 4-sample group's raw locations.
@@ -1611,29 +1640,22 @@ template <typename T, typename TL, bool SOFTMAX, int GP>
 __global__ __launch_bounds__(1024) void msda_record_sort_kernel(const Problem p, const BwdGeom bg, const Records rec) {
   using W = RecordWeight<T, SOFTMAX>;
   using LocWord = std::conditional_t<sizeof(TL) == 2, uint32_t, u32x2_v>;  // one location pair
-  __shared__ Level levels[kRecordLevels];
-  __shared__ LevelTiles lt[kRecordLevels];
-  __shared__ int64_t total;
-  __shared__ int first[kRecordLevels];
+  __shared__ RecordLevels plan;
   __shared__ int hist[kRecordKeys];
   __shared__ int scan_sums[1024 / kWave];
   extern __shared__ __align__(16) unsigned char stage[];
   const int T_ = int(blockDim.x), tid = int(threadIdx.x);
-  bool overlap = false;
-  const int64_t ntiles = load_tiles(p, bg, levels, lt, &total, &overlap);
-  if (overlap && p.zero_gv) zero_grad_value(p);
+  if (tid < kWave) plan_records(p, bg, rec, plan);
   if (blockIdx.x == 0)
     for (int i = tid; i < kXcds * kQueueLine; i += T_) rec.queue[i] = 0;
   int group, h;
-  if (ntiles < 0 || !xcd_group_block(p.H, p.B * rec.nch, &group, &h)) return;
+  const bool work = xcd_group_block(p.H, p.B * rec.nch, &group, &h);
   const int c = group % rec.nch, b = group / rec.nch;
   const int LP = p.L * p.P, gpq = LP / 4;
   const int q0 = c * rec.qc, nq = min(rec.qc, p.Q - q0);
   const int ngroups = nq * gpq;
   const int64_t unit0 = (int64_t(b) * p.Q + q0) * p.H + h;
   const int64_t bh = int64_t(b) * p.H + h;
-  const RecordBuckets bk = record_buckets(p, rec, lt, ntiles, first);
-  const int nkeys = bk.count;
 
   GroupLoc<TL> loc[GP];
   W wt[GP][4];
@@ -1644,7 +1666,7 @@ __global__ __launch_bounds__(1024) void msda_record_sort_kernel(const Problem p,
 #pragma unroll
     for (int k = 0; k < 4; ++k) key[i][k] = pos[i][k] = -1;
     ql[i] = 0;
-    if (g >= ngroups) continue;
+    if (!work || g >= ngroups) continue;
     const uint32_t q = fdiv(uint32_t(g), bg.div_gpq), r = uint32_t(g) - q * uint32_t(gpq);
     ql[i] = int(q);
     const int64_t unit = unit0 + int64_t(q) * p.H;
@@ -1677,6 +1699,10 @@ __global__ __launch_bounds__(1024) void msda_record_sort_kernel(const Problem p,
       __builtin_memcpy(wt[i], &a, sizeof(a));
     }
   }
+  __syncthreads();  // the plan; the loads above do not wait for it
+  if (plan.overlap && p.zero_gv) zero_grad_value(p);
+  if (!work) return;
+  const int nkeys = plan.buckets, shift = plan.shift;
   auto pair_of = [&](const GroupLoc<TL>& l, int k) __attribute__((always_inline)) -> LocWord {
     if constexpr (sizeof(TL) == 2) return l.w[0][k];
     else return LocWord{l.w[k / 2][2 * (k & 1)], l.w[k / 2][2 * (k & 1) + 1]};
@@ -1686,8 +1712,8 @@ __global__ __launch_bounds__(1024) void msda_record_sort_kernel(const Problem p,
     const int g = tid + i * T_;
     if (g >= ngroups) continue;
     const int l = int(fdiv(uint32_t(g) - uint32_t(ql[i]) * uint32_t(gpq), bg.div_gpl));
-    const Level lv = levels[l];
-    const LevelTiles tl = lt[l];
+    const Level lv = plan.level[l];
+    const LevelTiles tl = plan.tiles[l];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const LocWord v = pair_of(loc[i], k);
@@ -1700,7 +1726,7 @@ __global__ __launch_bounds__(1024) void msda_record_sort_kernel(const Problem p,
         y = __uint_as_float(v[1]);
       }
       const int kk = sample_key<float>(x, y, lv, tl);
-      key[i][k] = kk < 0 ? -1 : bk.shift < 0 ? record_bucket(kk) : first[l] + ((kk / 4 - tl.base) >> bk.shift);
+      key[i][k] = kk < 0 ? -1 : shift < 0 ? record_bucket(kk) : plan.first[l] + ((kk / 4 - tl.base) >> shift);
     }
   }
 
@@ -3315,9 +3341,16 @@ constexpr int record_owner_waves(int nb, int es) {
   return es == 4 ? (nb == 1 ? 12 : nb == 2 ? 8 : 4) : (nb <= 2 ? 12 : 8);
 }
 
-// When a level's tasks are split over a workgroup (K-blocks expected per task).
-constexpr float kSplitKBlocks = 3.f;  // and at least twice a wave's average work
-constexpr int kSplitRounds = 6;       // or this many K-blocks for every wave
+// A level's tasks are split over the workgroup from this many expected K-blocks per
+// task, and from this multiple of what a wave gets on average. Below, the merge and its
+// barriers cost more than the tasks' length: with splits from the average on, the owner
+// takes 53 instead of 35 us at B = 2, Q = 5,376 bf16 (a level of 8 K-blocks, average
+// 7.7), and 166 instead of 141 at five levels, H = 4, D = 64 (one of 54, average 46);
+// with splits only from 1.5 times it, 256 instead of 216 at B = 4, Q = 21,504 float
+// (110, average 74). Tasks of 4 K-blocks split: 48 instead of 43 us for 300 queries.
+constexpr float kSplitKBlocks = 5.f;
+constexpr float kSplitShare = 1.25f;
+constexpr int kLongTasks = 1 << 30;   // marks a count of longer tasks than that
 constexpr float kShortKBlocks = 2.f;  // a short task has at most this many, expected
 
 template <typename T, typename TL, int NB, bool SOFTMAX>
@@ -3331,32 +3364,75 @@ msda_record_owner_kernel(const Problem p, const BwdGeom bg, const Records rec, c
   constexpr size_t kRowsBytes = size_t(kMfmaK) * size_t(mfma_row_bytes(NB)) * (kSplit ? 2 : 1);
   constexpr size_t kWaveBytes = std::max(kRowsBytes + size_t(kMfmaTileBytes), size_t(4 * NB * kWave * 16));
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ Level levels[kRecordLevels];
-  __shared__ LevelTiles lt[kRecordLevels];
-  __shared__ int level_buckets[kRecordLevels];
-  __shared__ int64_t total;
-  __shared__ float work_s[kRecordLevels];        // expected K-blocks per task
+  __shared__ RecordLevels plan;
   __shared__ int order_s[kRecordLevels];         // levels, heaviest tasks first
   __shared__ int split_end_s[kRecordLevels], wave_end_s[kRecordLevels];  // list positions after each ordered level
+  __shared__ int counts_s[3];
   __shared__ int next_s[2];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uni(tid / kWave);
   const int LP = p.L * p.P;
   unsigned char* gst = smem + size_t(wave) * kWaveBytes;  // grad_out rows (hi, then lo)
   unsigned char* wt = gst + kRowsBytes;                   // eight weight tiles (hi, then lo)
+  const int xcd = int(blockIdx.x) % kXcds, slot = int(blockIdx.x) / kXcds;
+  const int slots = int(gridDim.x) / kXcds;
+  const int per_tile = p.B * p.H;
 
-  bool overlap;
-  const int64_t ntiles = load_tiles(p, bg, levels, lt, &total, &overlap);
+  // The plan and the lists, by the first wave, lane l for level l. A level's tasks are
+  // split over the workgroup when one is much longer than what a wave gets on average.
+  if (wave == 0) {
+    plan_records(p, bg, rec, plan);
+    wave_lds_order();
+    LevelTiles t{0, 0, 0, 0, 0};
+    if (lane < p.L) t = plan.tiles[lane];
+    const int n = t.ntx * t.nty;
+    const float side = float(1 << t.lw), straddle = (1.f + 1.f / side) * (1.f + 1.f / side);
+    const float w = n > 0 ? float(p.Q) * float(p.P) * straddle / (float(kMfmaK) * float(n)) : 0.f;
+    int rank = 0;
+    float all = 0.f;
+    for (int l = 0; l < p.L; ++l) {
+      const float o = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), l));
+      rank += o > w || (o == w && l < lane) ? 1 : 0;
+      all += o * float(__builtin_amdgcn_readlane(n, l));
+    }
+    const float average = all * float(per_tile) / (float(gridDim.x) * float(kWaves));
+    const bool split = w >= kSplitKBlocks && w >= kSplitShare * average;
+    const int64_t tasks = int64_t(n) * per_tile;
+    const int mine = int((xcd + 1) * tasks / kXcds - xcd * tasks / kXcds);
+    if (lane < p.L) {
+      order_s[rank] = lane;
+      split_end_s[rank] = split ? mine : 0;
+      wave_end_s[rank] = split ? 0 : mine | (w > kShortKBlocks ? kLongTasks : 0);
+    }
+    wave_lds_order();
+    const int a = lane < p.L ? split_end_s[lane] : 0, c = lane < p.L ? wave_end_s[lane] : 0;
+    const int sa = wave_inclusive_scan(a), sc = wave_inclusive_scan(c & ~kLongTasks);
+    if (lane < p.L) {
+      split_end_s[lane] = sa;
+      wave_end_s[lane] = sc;
+    }
+    const uint64_t longer = __ballot((c & kLongTasks) != 0);
+    const int last = longer ? 63 - __builtin_clzll(longer) : 0;
+    const int from = longer ? __builtin_amdgcn_readlane(sc, last) : 0;
+    if (lane == 0) {
+      counts_s[0] = __builtin_amdgcn_readlane(sa, kWave - 1);
+      counts_s[1] = __builtin_amdgcn_readlane(sc, kWave - 1);
+      counts_s[2] = from;
+    }
+  }
+  mfma_zero_tiles(wt, lane);
+  __syncthreads();
+  const int ntiles = plan.ntiles;
   // Overlapping levels: the sort zeroed grad_value, and the owners add.
-  const bool add = overlap;
+  const bool add = plan.overlap != 0;
   if (!accumulate && !add) {
     // grad_value at positions no valid level covers is zero (the tiles own the others).
     const int64_t n = int64_t(p.B) * p.S;
     for (int64_t idx = int64_t(blockIdx.x) * blockDim.x + tid; idx < n; idx += int64_t(gridDim.x) * blockDim.x) {
-      const int pos = int(idx % p.S);
+      const int pos = int(uint32_t(idx) % uint32_t(p.S));
       bool covered = false;
       for (int l = 0; l < p.L && !covered; ++l) {
-        const Level lv = levels[l];
-        covered = lv.ok && pos >= lv.start && int64_t(pos) < int64_t(lv.start) + int64_t(lv.h) * lv.w;
+        const Level lv = plan.level[l];
+        covered = lv.ok && pos >= lv.start && pos < lv.start + lv.h * lv.w;
       }
       if (!covered) {
         T* dst = reinterpret_cast<T*>(p.grad_value) + idx * p.H * D;
@@ -3365,60 +3441,11 @@ msda_record_owner_kernel(const Problem p, const BwdGeom bg, const Records rec, c
     }
   }
   if (ntiles <= 0) return;
-  const RecordBuckets bk = record_buckets(p, rec, lt, ntiles, level_buckets);
-
-  // The lists. A level's tasks are split over the workgroup when one is longer than
-  // twice what a wave gets on average, or so long that the merge does not matter.
-  const int xcd = int(blockIdx.x) % kXcds, slot = int(blockIdx.x) / kXcds;
-  const int slots = int(gridDim.x) / kXcds;
-  const int per_tile = p.B * p.H;
-  if (tid < p.L) {
-    const LevelTiles t = lt[tid];
-    const int n = t.ntx * t.nty;
-    const float side = float(1 << t.lw), straddle = (1.f + 1.f / side) * (1.f + 1.f / side);
-    work_s[tid] = n > 0 ? float(p.Q) * float(p.P) * straddle / (float(kMfmaK) * float(n)) : 0.f;
-  }
-  __syncthreads();
-  if (tid < p.L) {
-    int rank = 0;
-    float all = 0.f;
-    for (int l = 0; l < p.L; ++l) {
-      const float w = work_s[l];
-      rank += w > work_s[tid] || (w == work_s[tid] && l < tid) ? 1 : 0;
-      all += w * float(lt[l].ntx * lt[l].nty);
-    }
-    const float average = all * float(per_tile) / (float(gridDim.x) * float(kWaves));
-    const float w = work_s[tid];
-    const bool split = w >= kSplitKBlocks && w >= 2.f * average || w >= float(kSplitRounds * kWaves);
-    const int64_t n = int64_t(lt[tid].ntx * lt[tid].nty) * per_tile;
-    const int mine = int((xcd + 1) * n / kXcds - xcd * n / kXcds);
-    order_s[rank] = tid;
-    split_end_s[rank] = split ? mine : 0;
-    wave_end_s[rank] = split ? 0 : mine;
-  }
-  __syncthreads();
-  int nsplit = 0, nwave = 0, short_from = 0;
-  for (int i = 0; i < p.L; ++i) {
-    nsplit += split_end_s[i];
-    nwave += wave_end_s[i];
-    if (work_s[order_s[i]] > kShortKBlocks) short_from = nwave;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int a = 0, b = 0;
-    for (int i = 0; i < p.L; ++i) {
-      split_end_s[i] = a += split_end_s[i];
-      wave_end_s[i] = b += wave_end_s[i];
-    }
-  }
-  __syncthreads();
-  nsplit = uni(nsplit);
-  nwave = uni(nwave);
+  const int nsplit = uni(counts_s[0]), nwave = uni(counts_s[1]), short_from = uni(counts_s[2]);
   int* split_queue = rec.queue + xcd * kQueueLine;
   int* wave_queue = split_queue + 1;
   const int g16 = lane >> 4, i16 = lane & 15;
   T* gv = reinterpret_cast<T*>(p.grad_value);
-  mfma_zero_tiles(wt, lane);
 
   // One task: its K-blocks kb0, kb0 + kbstep, ... into acc.
   struct Task {
@@ -3428,7 +3455,8 @@ msda_record_owner_kernel(const Problem p, const BwdGeom bg, const Records rec, c
   };
   // The task at position k of a list, and its candidate source.
   RecordSource<T, TL, SOFTMAX> src;
-  src.row = uint32_t(bk.count + 1);
+  src.row = uint32_t(uni(plan.buckets) + 1);
+  const int shift = uni(plan.shift);
   src.nch = rec.nch;
   src.qc = rec.qc;
   src.LP = LP;
@@ -3438,9 +3466,9 @@ msda_record_owner_kernel(const Problem p, const BwdGeom bg, const Records rec, c
     int oi = 0;
     while (oi + 1 < p.L && k >= ends[oi]) ++oi;
     const int l = uni(order_s[oi]);
-    Level lv = levels[l];
+    Level lv = plan.level[l];
     lv = Level{uni(lv.h), uni(lv.w), uni(lv.start), uni(lv.ok)};
-    LevelTiles tl = lt[l];
+    LevelTiles tl = plan.tiles[l];
     tl = LevelTiles{uni(tl.lh), uni(tl.lw), uni(tl.ntx), uni(tl.nty), uni(tl.base)};
     const int ntl = tl.ntx * tl.nty;
     const int64_t n = int64_t(ntl) * per_tile;
@@ -3467,7 +3495,7 @@ msda_record_owner_kernel(const Problem p, const BwdGeom bg, const Records rec, c
     src.w = reinterpret_cast<const RecordWeight<T, SOFTMAX>*>(rec.w) + first;
     src.q = rec.q + first;
     src.offs = rec.offs + bh * rec.nch * src.row;
-    const uint32_t first_bucket = uint32_t(uni(level_buckets[l]));
+    const uint32_t first_bucket = uint32_t(uni(plan.first[l]));
 #pragma unroll
     for (int st = 0; st < 4; ++st)
 #pragma unroll
@@ -3475,7 +3503,7 @@ msda_record_owner_kernel(const Problem p, const BwdGeom bg, const Records rec, c
     parts = 0;
     auto groups = [&]<int NST>() __attribute__((always_inline)) {
       for (int g = 0; g < src.nch; g += kRecordGroup) {
-        src.group(g, first_bucket, tile, tl.ntx, ty, bk.shift);
+        src.group(g, first_bucket, tile, tl.ntx, ty, shift);
         parts = max(parts, int((src.ncand + kMfmaK - 1) / kMfmaK));
         mfma_tile_kblocks<T, NB, NST>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
       }
