@@ -344,6 +344,31 @@ __device__ inline void atomic_add_channels(char* p, typename Elem<T>::acc w, con
 }
 
 
+// Unsigned 32-bit division by a divisor fixed per launch: one multiply-high, an
+// add and two shifts (Granlund and Montgomery, "Division by invariant integers
+// using multiplication", 1994, section 4) instead of the ~30-instruction software
+// division. Exact for every dividend below 2^32.
+struct FastDiv {
+  uint32_t d, m;
+  int s;
+};
+
+FastDiv make_fastdiv(uint32_t d) {
+  FastDiv f{d, 0u, 0};
+  if (d <= 1) return f;
+  int l = 0;
+  while ((uint64_t(1) << l) < d) ++l;  // ceil(log2 d)
+  f.m = uint32_t(((uint64_t(1) << 32) * ((uint64_t(1) << l) - d)) / d + 1);
+  f.s = l - 1;
+  return f;
+}
+
+__device__ inline uint32_t fdiv(uint32_t n, const FastDiv& f) {
+  if (f.d <= 1) return n;
+  const uint32_t t = __umulhi(f.m, n);
+  return (t + ((n - t) >> 1)) >> f.s;
+}
+
 // ---------------------------------------------------------------------------
 // Problem description, passed by value to every kernel.
 
@@ -365,6 +390,9 @@ struct Problem {
   int blocks_per_batch;
   int num_blocks;
   int loc_piece, attn_piece;  // bytes per lane access copying a wave's records to LDS
+  int chunk;                  // samples of a unit staged at once
+  int loc_pair;               // grad_loc takes a float pair in one 8-byte store
+  FastDiv div_p;              // by P
   int atomic_gv;              // backward: grad_sample scatters grad_value with atomics
   // Backward on the matrix-core owners: levels that share positions of S are sorted
   // too (each level's tiles are its own buckets); the count pass zeroes grad_value
@@ -619,22 +647,16 @@ __device__ inline char* row_at(char* img, uint32_t row, uint32_t row_bytes, uint
   return img + (uint64_t(row) * row_bytes + lane_bytes);
 }
 
-// Phase 1, shared by both directions: stage every sample of the lane's unit and
-// return the unit's softmax statistics (max and 1 / sum of exp), if any.
-template <typename T, typename TL, bool SOFTMAX>
-__device__ inline void stage_samples(const Problem& p, const LaneMap& m, const Level* levels,
-                                     const UnitRaw& raw, Staged<typename Elem<T>::acc>* wst,
-                                     typename Elem<T>::acc& smax,
-                                     typename Elem<T>::acc& sinv,
-                                     typename Elem<T>::acc* ssum = nullptr) {
+// A unit's softmax statistics over its L * P logits (max, 1 / sum of exp, and the sum),
+// by all its lanes; (0, 1) for the linear method.
+template <typename T, bool SOFTMAX>
+__device__ inline void unit_softmax(const LaneMap& m, int LP, const UnitRaw& raw, typename Elem<T>::acc& smax,
+                                    typename Elem<T>::acc& sinv, typename Elem<T>::acc* ssum = nullptr) {
   using A = typename Elem<T>::acc;
-  constexpr int ES = Elem<T>::size;
-  const int LP = p.L * p.P;
-  const TL* loc = reinterpret_cast<const TL*>(raw.loc);
-  const T* attn = reinterpret_cast<const T*>(raw.attn);
   smax = A(0);
   sinv = A(1);
   if constexpr (SOFTMAX) {
+    const T* attn = reinterpret_cast<const T*>(raw.attn);
     A mx = -INFINITY;
     if (m.unit_ok)
       for (int s = m.t; s < LP; s += m.lh) mx = fmax(mx, load_acc(attn + s));
@@ -647,10 +669,25 @@ __device__ inline void stage_samples(const Problem& p, const LaneMap& m, const L
     sinv = A(1) / sum;
     if (ssum) *ssum = sum;
   }
+}
+
+// Phase 1, shared by both directions: stage samples s0 .. s0 + n - 1 of the lane's unit
+// (a chunk: all of them, where a wave's records are few). FAST: the level of a sample by
+// multiplication (grad_sample, 26.6 against 27.4 us at B = 2, Q = 5,376 bf16; the
+// forward loses 0.2 us to the extra kernel arguments in calls of 6 us).
+template <typename T, typename TL, bool SOFTMAX, bool FAST>
+__device__ inline void stage_samples(const Problem& p, const LaneMap& m, const Level* levels, const UnitRaw& raw,
+                                     Staged<typename Elem<T>::acc>* wst, int s0, int n,
+                                     typename Elem<T>::acc smax, typename Elem<T>::acc sinv) {
+  using A = typename Elem<T>::acc;
+  const TL* loc = reinterpret_cast<const TL*>(raw.loc);
+  const T* attn = reinterpret_cast<const T*>(raw.attn);
   if (!m.unit_ok) return;
-  for (int s = m.t; s < LP; s += m.lh) {
+  for (int i = m.t; i < n; i += m.lh) {
+    const int s = s0 + i;
     const Geom<A> g = geometry<A>(load_acc(loc + 2 * s), load_acc(loc + 2 * s + 1),
-                                  levels[s / p.P], uint32_t(m.h), uint32_t(p.H));
+                                  levels[FAST ? int(fdiv(uint32_t(s), p.div_p)) : s / p.P], uint32_t(m.h),
+                                  uint32_t(p.H));
     A a = load_acc(attn + s);
     if constexpr (SOFTMAX) a = exp_acc(a - smax) * sinv;
     Staged<A> st;
@@ -662,14 +699,18 @@ __device__ inline void stage_samples(const Problem& p, const LaneMap& m, const L
     st.w[1] = g.m01 ? g.w01 * a : A(0);
     st.w[2] = g.m10 ? g.w10 * a : A(0);
     st.w[3] = g.m11 ? g.w11 * a : A(0);
-    wst[s * m.uw_count + m.uw] = st;
+    wst[i * m.uw_count + m.uw] = st;
   }
 }
 
 // ---------------------------------------------------------------------------
 // Forward.
 
-template <typename T, typename TL, int CV, bool SOFTMAX>
+// CHUNKED: a unit's samples are staged p.chunk at a time, where all of them would take
+// so much LDS that it limits the waves per CU. For 40 samples a unit (B = 3, Q = 9,835,
+// H = 4, D = 64 bf16) the forward takes 90 instead of 102 us; for 12 and 16 samples the
+// loop over chunks costs 3-4 % in float and gains nothing in 16 bits.
+template <typename T, typename TL, int CV, bool SOFTMAX, bool CHUNKED>
 __global__ __launch_bounds__(kWave * kMaxWavesPerBlock) void msda_forward_kernel(const Problem p) {
   using A = typename Elem<T>::acc;
   constexpr int ES = Elem<T>::size;
@@ -678,16 +719,22 @@ __global__ __launch_bounds__(kWave * kMaxWavesPerBlock) void msda_forward_kernel
   const LaneMap m = map_lane(p);
   const int LP = p.L * p.P;
   constexpr size_t kRec = sizeof(Staged<A>);
-  Staged<A>* wst = reinterpret_cast<Staged<A>*>(smem + sizeof(Level) * p.L + kRec * m.wave * m.uw_count * LP);
-  const size_t raw_at = (sizeof(Level) * p.L + kRec * (blockDim.x / kWave) * m.uw_count * LP + 15) & ~size_t(15);
+  const int staged = CHUNKED ? p.chunk : LP;
+  Staged<A>* wst = reinterpret_cast<Staged<A>*>(smem + sizeof(Level) * p.L + kRec * m.wave * m.uw_count * staged);
+  const size_t raw_at =
+      (sizeof(Level) * p.L + kRec * (blockDim.x / kWave) * m.uw_count * staged + 15) & ~size_t(15);
   const UnitRaw raw = copy_unit_records<T, TL>(p, m, smem + raw_at);
   load_levels(p, levels);
   __syncthreads();
   A smax, sinv;
-  stage_samples<T, TL, SOFTMAX>(p, m, levels, raw, wst, smax, sinv);
-  __syncthreads();
+  unit_softmax<T, SOFTMAX>(m, LP, raw, smax, sinv);
 
-  if (!m.unit_ok || m.t * CV >= p.D) return;
+  if constexpr (!CHUNKED) {
+    stage_samples<T, TL, SOFTMAX, false>(p, m, levels, raw, wst, 0, LP, smax, sinv);
+    __syncthreads();
+    if (!m.unit_ok || m.t * CV >= p.D) return;
+  }
+  const bool lane_ok = m.unit_ok && m.t * CV < p.D;
   const char* img = p.value + int64_t(m.b) * p.S * p.H * p.D * ES;
   const uint32_t row_bytes = uint32_t(p.D * ES), lane_bytes = uint32_t(m.t * CV * ES);
   A acc[CV];
@@ -696,8 +743,7 @@ __global__ __launch_bounds__(kWave * kMaxWavesPerBlock) void msda_forward_kernel
   // Every corner value is widened to the accumulation type and multiplied by its
   // weight (attention * bilinear, kept in that type) into the sum, as the
   // reference's kernels do with their fp32 accumulator.
-#pragma unroll 2
-  for (int s = 0; s < LP; ++s) {
+  auto add_sample = [&](int s) __attribute__((always_inline)) {
     const Staged<A> st = wst[s * m.uw_count + m.uw];
     A v[4][CV];
 #pragma unroll
@@ -706,6 +752,22 @@ __global__ __launch_bounds__(kWave * kMaxWavesPerBlock) void msda_forward_kernel
     for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int i = 0; i < CV; ++i) acc[i] = fma(st.w[c], v[c][i], acc[i]);
+  };
+  if constexpr (CHUNKED) {
+    for (int s0 = 0; s0 < LP; s0 += p.chunk) {
+      const int n = min(p.chunk, LP - s0);
+      wave_lds_order();  // after the previous chunk's reads
+      stage_samples<T, TL, SOFTMAX, false>(p, m, levels, raw, wst, s0, n, smax, sinv);
+      wave_lds_order();
+      if (lane_ok) {
+#pragma unroll 2
+        for (int s = 0; s < n; ++s) add_sample(s);
+      }
+    }
+    if (!lane_ok) return;
+  } else {
+#pragma unroll 2
+    for (int s = 0; s < LP; ++s) add_sample(s);
   }
   Chan<T, CV>::store(p.out + (m.gunit * p.D + m.t * CV) * ES, acc);
 }
@@ -781,31 +843,6 @@ constexpr int kMaxOrderedLevels = 64;
 // counters, each on its own 128-byte line (plus the slack to align the first).
 constexpr int kQueueLine = 32;
 constexpr int kQueueInts = (kXcds + 1) * kQueueLine;
-
-// Unsigned 32-bit division by a divisor fixed per launch: one multiply-high, an
-// add and two shifts (Granlund and Montgomery, "Division by invariant integers
-// using multiplication", 1994, section 4) instead of the ~30-instruction software
-// division. Exact for every dividend below 2^32.
-struct FastDiv {
-  uint32_t d, m;
-  int s;
-};
-
-FastDiv make_fastdiv(uint32_t d) {
-  FastDiv f{d, 0u, 0};
-  if (d <= 1) return f;
-  int l = 0;
-  while ((uint64_t(1) << l) < d) ++l;  // ceil(log2 d)
-  f.m = uint32_t(((uint64_t(1) << 32) * ((uint64_t(1) << l) - d)) / d + 1);
-  f.s = l - 1;
-  return f;
-}
-
-__device__ inline uint32_t fdiv(uint32_t n, const FastDiv& f) {
-  if (f.d <= 1) return n;
-  const uint32_t t = __umulhi(f.m, n);
-  return (t + ((n - t) >> 1)) >> f.s;
-}
 
 struct BwdGeom {
   int cap;          // positions per tile at most (power of two)
@@ -3635,11 +3672,14 @@ __device__ inline void corner_dots(const LaneMap& m, Staged<typename Elem<T>::ac
 }
 
 // A location gradient pair: one 4-byte store for 16-bit locations (grad_loc is
-// 4-byte aligned), else one store per coordinate.
+// 4-byte aligned), one 8-byte store for float ones where grad_loc is aligned for it
+// (`pair`), else one store per coordinate.
 template <typename TL, typename A>
-__device__ inline void store_loc_pair(TL* p, A x, A y) {
+__device__ inline void store_loc_pair(TL* p, A x, A y, int pair) {
   if constexpr (sizeof(TL) == 2) {
     *reinterpret_cast<uint32_t*>(p) = Chan16<TL, 2>::pack(x, y);
+  } else if (sizeof(TL) == 4 && pair) {  // uniform
+    *reinterpret_cast<u32x2_v*>(p) = u32x2_v{__float_as_uint(float(x)), __float_as_uint(float(y))};
   } else {
     store_elem(p, x);
     store_elem(p + 1, y);
@@ -3656,9 +3696,9 @@ __global__ __launch_bounds__(kWave * kMaxWavesPerBlock) void msda_grad_sample_ke
   const LaneMap m = map_lane(p);
   const int LP = p.L * p.P;
   Staged<A>* wst = reinterpret_cast<Staged<A>*>(smem + sizeof(Level) * p.L) +
-                   m.wave * m.uw_count * LP;
+                   m.wave * m.uw_count * p.chunk;
   const size_t raw_at =
-      (sizeof(Level) * p.L + sizeof(Staged<A>) * (blockDim.x / kWave) * m.uw_count * LP + 15) & ~size_t(15);
+      (sizeof(Level) * p.L + sizeof(Staged<A>) * (blockDim.x / kWave) * m.uw_count * p.chunk + 15) & ~size_t(15);
   const UnitRaw raw = copy_unit_records<T, TL>(p, m, smem + raw_at);
 
   if (threadIdx.x == 0) *overlap_flag() = 0;
@@ -3666,7 +3706,7 @@ __global__ __launch_bounds__(kWave * kMaxWavesPerBlock) void msda_grad_sample_ke
   __syncthreads();
   overlap_flag_raise(levels, p.L);
   A smax, sinv, ssum = A(1);
-  stage_samples<T, TL, SOFTMAX>(p, m, levels, raw, wst, smax, sinv, &ssum);
+  unit_softmax<T, SOFTMAX>(m, LP, raw, smax, sinv, &ssum);
   if constexpr (SOFTMAX)  // the unit's log-sum-exp for the grad_value kernel, as msda_softmax_stats_kernel's
     if (p.stats && m.unit_ok && m.t == 0) reinterpret_cast<SoftStat<A>*>(p.stats)[m.gunit] = SoftStat<A>{smax + log(ssum)};
   __syncthreads();
@@ -3684,56 +3724,72 @@ __global__ __launch_bounds__(kWave * kMaxWavesPerBlock) void msda_grad_sample_ke
   const uint32_t row_bytes = uint32_t(p.D * ES), lane_bytes = uint32_t(m.t * CV * ES);
   R g{};
   if (lane_ok) g = *reinterpret_cast<const R*>(p.grad_out + (m.gunit * p.D + m.t * CV) * ES);
-  if (gv_img != nullptr && lane_ok) {
-    // Each lane adds weight * grad_out into its channels of every corner with a
-    // non-zero weight, with global atomics (before the dots overwrite the weights).
-    A gw[CV];
-    Chan<T, CV>::from_raw(g, gw);
-    for (int s = 0; s < LP; ++s) {
-      const Staged<A> st = wst[s * m.uw_count + m.uw];
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if (st.w[c] != A(0))
-          atomic_add_channels<T, CV>(row_at(gv_img, st.off[c], row_bytes, lane_bytes), st.w[c], gw);
-    }
-  }
-  int s = 0;
-  for (; s + kSampleBatch <= LP; s += kSampleBatch)
-    corner_dots<T, CV, kSampleBatch>(m, wst, s, lane_ok, img, row_bytes, lane_bytes, g);
-  for (; s < LP; ++s) corner_dots<T, CV, 1>(m, wst, s, lane_ok, img, row_bytes, lane_bytes, g);
-  wave_lds_order();  // other lanes of the unit stored some of a sample's sums
-
-  // Per-sample location and weight gradients by the lane that staged the sample.
   const TL* loc = reinterpret_cast<const TL*>(raw.loc);
   const T* attn = reinterpret_cast<const T*>(raw.attn);
+  // Softmax: a sample's weight gradient takes the place of its location in the wave's
+  // copy, until the unit's sum is known.
+  A* gpvs = reinterpret_cast<A*>(const_cast<unsigned char*>(raw.loc));
+  constexpr int kGpv = 2 * int(sizeof(TL)) / int(sizeof(A));  // accumulators per location pair
   TL* gloc = reinterpret_cast<TL*>(p.grad_loc) + m.gunit * LP * 2;
   T* gattn = reinterpret_cast<T*>(p.grad_attn) + m.gunit * LP;
   A dot(0);
-  if (m.unit_ok) {
-    for (int s = m.t; s < LP; s += m.lh) {
-      const Level lv = levels[s / p.P];
-      const Geom<A> ge = geometry<A>(load_acc(loc + 2 * s), load_acc(loc + 2 * s + 1), lv, 0u, 1u);
-      A a = load_acc(attn + s);
-      if constexpr (SOFTMAX) a = exp_acc(a - smax) * sinv;
-      Staged<A>* slot = wst + s * m.uw_count + m.uw;
-      A gx, gy, gpv;
-      sample_grads<A>(ge, a, lv, slot->w[0], slot->w[1], slot->w[2], slot->w[3], &gx, &gy, &gpv);
-      store_loc_pair(gloc + 2 * s, gx, gy);
-      if constexpr (SOFTMAX) {
-        dot += a * gpv;
-        slot->w[0] = gpv;
-      } else {
-        store_elem(gattn + s, gpv);
+  for (int s0 = 0; s0 < LP; s0 += p.chunk) {
+    const int n = min(p.chunk, LP - s0);
+    wave_lds_order();  // after the previous chunk's reads
+    stage_samples<T, TL, SOFTMAX, true>(p, m, levels, raw, wst, s0, n, smax, sinv);
+    // One or two chunks: in step, so that the workgroup's waves read the same samples'
+    // rows together (B = 4, Q = 21,504 bf16: 128 against 131 us; with more chunks the
+    // barriers cost more, 96 against 92 us for 40 samples a unit).
+    if (LP <= 2 * p.chunk) __syncthreads();  // uniform
+    wave_lds_order();
+    if (gv_img != nullptr && lane_ok) {
+      // Each lane adds weight * grad_out into its channels of every corner with a
+      // non-zero weight, with global atomics (before the dots overwrite the weights).
+      A gw[CV];
+      Chan<T, CV>::from_raw(g, gw);
+      for (int s = 0; s < n; ++s) {
+        const Staged<A> st = wst[s * m.uw_count + m.uw];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (st.w[c] != A(0))
+            atomic_add_channels<T, CV>(row_at(gv_img, st.off[c], row_bytes, lane_bytes), st.w[c], gw);
+      }
+    }
+    int i = 0;
+    for (; i + kSampleBatch <= n; i += kSampleBatch)
+      corner_dots<T, CV, kSampleBatch>(m, wst, i, lane_ok, img, row_bytes, lane_bytes, g);
+    for (; i < n; ++i) corner_dots<T, CV, 1>(m, wst, i, lane_ok, img, row_bytes, lane_bytes, g);
+    wave_lds_order();  // other lanes of the unit stored some of a sample's sums
+
+    // Per-sample location and weight gradients by the lane that staged the sample.
+    if (m.unit_ok) {
+      for (int i = m.t; i < n; i += m.lh) {
+        const int s = s0 + i;
+        const Level lv = levels[fdiv(uint32_t(s), p.div_p)];
+        const Geom<A> ge = geometry<A>(load_acc(loc + 2 * s), load_acc(loc + 2 * s + 1), lv, 0u, 1u);
+        A a = load_acc(attn + s);
+        if constexpr (SOFTMAX) a = exp_acc(a - smax) * sinv;
+        const Staged<A>* slot = wst + i * m.uw_count + m.uw;
+        A gx, gy, gpv;
+        sample_grads<A>(ge, a, lv, slot->w[0], slot->w[1], slot->w[2], slot->w[3], &gx, &gy, &gpv);
+        store_loc_pair(gloc + 2 * s, gx, gy, p.loc_pair);
+        if constexpr (SOFTMAX) {
+          dot += a * gpv;
+          gpvs[s * kGpv] = gpv;
+        } else {
+          store_elem(gattn + s, gpv);
+        }
       }
     }
   }
   if constexpr (SOFTMAX) {
     dot = unit_sum(dot, m.lh);
     if (m.unit_ok) {
+      // The chunk is a multiple of the unit's lanes: s = t, t + lh, ... are the samples
+      // this lane staged.
       for (int s = m.t; s < LP; s += m.lh) {
         const A a = exp_acc(load_acc(attn + s) - smax) * sinv;
-        const A gpv = wst[s * m.uw_count + m.uw].w[0];
-        store_elem(gattn + s, a * (gpv - dot));
+        store_elem(gattn + s, a * (gpvs[s * kGpv] - dot));
       }
     }
   }
@@ -3789,8 +3845,17 @@ const char* dtype_name(int dtype) {
   }
 }
 
+// LDS bytes of one wave's staged records beyond which its units' samples are staged in
+// chunks (see msda_forward_kernel; grad_sample, which also takes fewer registers so, gains
+// from 12 samples a unit on: 133 against 136 us at B = 4, Q = 21,504 bf16, 26 against 29 at
+// B = 2, Q = 5,376, 93 against 120 for 40 samples; float's 3 KB for 12 stay whole, 238
+// against 257 us in chunks of 8).
+constexpr int64_t kChunkBytesForward = 8192;
+constexpr int64_t kChunkBytesBackward = 4096;
+
 struct Plan {
   int cv, lh_log2, waves, units_per_block, blocks_per_batch;
+  int chunk;  // samples of a unit staged at once: all, or a multiple of its lanes
   int64_t num_blocks;
   size_t lds;
 };
@@ -3838,9 +3903,15 @@ int make_plan(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t Q, 
   // and weights. When one wave's units do not fit, a unit takes more lanes (the
   // lanes past the channels stage samples and idle in the gathers), so a wave holds
   // fewer units.
+  auto chunk_for = [&](int lhl) {
+    const int64_t lh = int64_t(1) << lhl, bytes = (int64_t(kWave) >> lhl) * L * P * int64_t(staged);
+    const int64_t most = backward ? kChunkBytesBackward : kChunkBytesForward;
+    const int64_t n = (bytes + most - 1) / most;
+    return n <= 1 ? L * P : std::min<int64_t>(L * P, ((L * P + n - 1) / n + lh - 1) / lh * lh);
+  };
   auto lds_for = [&](int lhl, int w) {
     const int u = kWave >> lhl;
-    const size_t per_wave = size_t(u) * size_t(L * P) * staged;
+    const size_t per_wave = size_t(u) * size_t(chunk_for(lhl)) * staged;
     const size_t raw_wave = size_t(unit_raw_bytes(u, int(L * P), loc_es, es));
     return ((levels_bytes + per_wave * w + 15) & ~size_t(15)) + raw_wave * w;
   };
@@ -3862,6 +3933,7 @@ int make_plan(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t Q, 
   }
   plan->cv = cv;
   plan->lh_log2 = lh_log2;
+  plan->chunk = int(chunk_for(lh_log2));
   plan->waves = waves;
   plan->units_per_block = waves * uw;
   plan->blocks_per_batch = int((units + plan->units_per_block - 1) / plan->units_per_block);
@@ -4426,6 +4498,8 @@ Problem make_problem(const void* value, const void* shapes, const void* starts, 
   p.lh_log2 = plan.lh_log2;
   p.units_per_block = plan.units_per_block;
   p.blocks_per_batch = plan.blocks_per_batch;
+  p.chunk = plan.chunk;
+  p.div_p = make_fastdiv(uint32_t(P));
   p.num_blocks = int(plan.num_blocks);
   return p;
 }
@@ -4633,10 +4707,12 @@ int msda_forward(const void* value, int value_dtype, const void* spatial_shapes,
       value_dtype, loc_dtype == MSDA_F32 && value_dtype != MSDA_F32, plan.cv,
       [&]<typename T, typename TL, int CV>() {
         const dim3 grid(unsigned(plan.num_blocks)), block(unsigned(kWave * plan.waves));
-        if (softmax)
-          hipLaunchKernelGGL((msda_forward_kernel<T, TL, CV, true>), grid, block, plan.lds, st, p);
-        else
-          hipLaunchKernelGGL((msda_forward_kernel<T, TL, CV, false>), grid, block, plan.lds, st, p);
+        const bool chunked = plan.chunk < levels * points;
+        auto k = softmax ? (chunked ? msda_forward_kernel<T, TL, CV, true, true>
+                                    : msda_forward_kernel<T, TL, CV, true, false>)
+                         : (chunked ? msda_forward_kernel<T, TL, CV, false, true>
+                                    : msda_forward_kernel<T, TL, CV, false, false>);
+        hipLaunchKernelGGL(k, grid, block, plan.lds, st, p);
         return hipGetLastError();
       });
   if (err != hipSuccess)
@@ -4716,6 +4792,7 @@ static int backward_call(const void* value, int value_dtype, const void* spatial
   p.grad_loc = static_cast<char*>(grad_sampling_locations);
   p.grad_attn = static_cast<char*>(grad_attention_weights);
   p.atomic_gv = atomic_gv ? 1 : 0;
+  p.loc_pair = loc_dtype == MSDA_F32 && aligned(grad_sampling_locations, 8) ? 1 : 0;
   // The matrix-core owners take overlapping levels when nothing falls back to the
   // VALU owner kernel (which stores, and stands aside on overlap).
   p.sort_overlap = plan.bucket && plan.mfma && !plan.mfma_fallback && !atomic_gv ? 1 : 0;
