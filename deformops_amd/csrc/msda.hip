@@ -3926,20 +3926,22 @@ int make_plan(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t Q, 
     const int64_t n = (bytes + most - 1) / most;
     return n <= 1 ? L * P : std::min<int64_t>(L * P, ((L * P + n - 1) / n + lh - 1) / lh * lh);
   };
-  auto lds_for = [&](int lhl, int w) {
+  auto lds_for = [&](int lhl, int w, int64_t chunk) {
     const int u = kWave >> lhl;
-    const size_t per_wave = size_t(u) * size_t(chunk_for(lhl)) * staged;
+    const size_t per_wave = size_t(u) * size_t(chunk) * staged;
     const size_t raw_wave = size_t(unit_raw_bytes(u, int(L * P), loc_es, es));
     return ((levels_bytes + per_wave * w + 15) & ~size_t(15)) + raw_wave * w;
   };
-  while (lh_log2 < 6 && lds_for(lh_log2, 1) > kMaxLds) ++lh_log2;
-  const int uw = kWave >> lh_log2;
-  auto lds_of = [&](int w) { return lds_for(lh_log2, w); };
-  if (lds_of(1) > kMaxLds)
+  // Chunks change neither the lanes nor the limit: both go by the samples staged whole.
+  auto whole = [&] { return lds_for(lh_log2, 1, L * P); };
+  while (lh_log2 < 6 && whole() > kMaxLds) ++lh_log2;
+  if (whole() > kMaxLds)
     return fail(MSDA_ERR_UNSUPPORTED,
                 "msda: %lld samples per (query, head) do not fit the %zu-byte LDS staging of one "
                 "wave (%zu bytes needed)",
-                (long long)(L * P), kMaxLds, lds_of(1));
+                (long long)(L * P), kMaxLds, whole());
+  const int uw = kWave >> lh_log2;
+  auto lds_of = [&](int w) { return lds_for(lh_log2, w, chunk_for(lh_log2)); };
   const int64_t units = Q * H;
   int waves = kMaxWavesPerBlock;
   // Fewer waves per workgroup when the grid would leave CUs idle or LDS is short.

@@ -191,6 +191,22 @@ def test_launch_geometry_widens_units_whose_samples_overflow_a_wave(lib):
     assert "lds" in lib.cdll.msda_last_error().decode().lower()
 
 
+@pytest.mark.parametrize("backward", [False, True], ids=["forward", "backward"])
+@pytest.mark.parametrize(("dtype", "staged", "size"), [(0, 32, 4), (1, 32, 2), (2, 32, 2), (3, 48, 8)],
+                         ids=["f32", "f16", "bf16", "f64"])
+def test_launch_geometry_takes_as_many_samples_as_fit_one_wave_whole(lib, dtype, staged, size, backward):
+    # One unit's records, locations and weights, each region rounded up to 16 bytes, in
+    # 64 KiB: the same bound where the samples are staged in chunks.
+    def fits(n):
+        up = lambda b: (b + 15) // 16 * 16  # noqa: E731
+        return up(16 + n * staged) + up(n * 2 * size) + up(n * size) <= 64 * 1024
+
+    most = max(n for n in range(1, 4096) if fits(n))
+    for samples in (most, most + 1):
+        rc, *_ = geometry(lib, dtype, (1, 64, 1, 8, 16, 1, samples), backward)
+        assert rc == (0 if fits(samples) else 2), samples
+
+
 @pytest.mark.parametrize(
     ("levels", "points", "dtype", "head_dim", "expected"),
     [
