@@ -502,9 +502,9 @@ def main() -> int:
             # request rate of their row gathers (forward, grad_sample) and the latency
             # of grad_value's scattered candidate reads: "binding" and "l2_requests".
             "bound": "hbm",
-            "binding": "l2_request_rate (forward, grad_sample); memory latency (grad_value)",
-            "kernel": "one msda_forward + msda_backward_workspace C-ABI call pair (forward kernel, bucket sort, "
-                      "grad_value, grad_sample beside the sort on a side stream), on one caller stream",
+            "binding": "l2_request_rate (forward, grad_sample); lds (grad_value)",
+            "kernel": "one msda_forward + msda_backward_workspace C-ABI call pair (forward kernel, record sort, "
+                      "grad_value owners, grad_sample), on one caller stream",
             "achieved": round(call_gbs, 1),
             "peak": PEAK_HBM_GBS,
             "unit": "GB/s",

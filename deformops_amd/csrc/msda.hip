@@ -778,8 +778,17 @@ __global__ __launch_bounds__(kWave * kMaxWavesPerBlock) void msda_forward_kernel
 // grad_value is computed owner-side: every element has exactly one writer, which
 // sums its contributions in fp32 (fp64 for double) registers and stores once, so
 // there are no atomics on grad_value, no zero-fill and no float32 copy. The
-// location and weight gradients are sample-parallel like the forward. Kernels, in
-// stream order:
+// location and weight gradients are sample-parallel like the forward.
+//
+// A workspace call with P a multiple of 4 (backward_call has the other conditions) runs
+// three kernels, each described where it stands:
+//
+//   msda_record_sort_kernel    Every chunk of queries sorted in LDS into location, weight
+//                              and query streams, in bucket order.
+//   msda_record_owner_kernel   The tile owners on the matrix cores, reading the streams.
+//   msda_grad_sample_kernel    Location and weight gradients, over the streams.
+//
+// Other calls sort sample indices instead. Their kernels, in stream order:
 //
 //   msda_bucket_kernel<COUNT>  Counting sort of the samples of every (b, h) by the
 //   msda_bucket_scan_kernel    level tile that holds their top-left corner (tiles

@@ -154,19 +154,27 @@ int msda_backward(const void* value, int value_dtype,
 /*
  * msda_backward with a caller workspace of at least msda_backward_workspace_size
  * bytes for the same sizes (device memory, 256-byte aligned; its contents are
- * ignored and left undefined). Writes the same three gradients. The bucket sort keeps
- * its counters and sorted sample indices in the workspace instead of
- * grad_attention_weights and grad_sampling_locations, so the location and weight
- * gradient kernel no longer has to run after it: where that kernel adds nothing into
- * grad_value (the matrix-core owners take every level, overlapping ones included,
- * and MSDA_GRAD_VALUE_ATOMIC is off) and the call has at least 2^21 samples, the call
- * forks it onto a side stream of the calling thread (created on the first such call
- * per thread and device, default priority) beside the sort and the grad_value
- * kernel, and joins the caller's stream at the end of the call (with MSDA_SOFTMAX,
- * before the grad_value kernel, which then reads the softmax statistics grad_sample
- * leaves): 9-13 us less GPU time at B = 4, Q = 21,504 in bf16, 21 us with softmax.
- * The fork and join cost the calling thread about 45 us, so smaller calls, whose
- * GPU time would not hide that, keep one stream.
+ * ignored and left undefined). Writes the same three gradients.
+ *
+ * Where P is a multiple of 4, L at most 16, an image under 2^20 positions, the matrix
+ * cores take grad_value (16-bit or float values, D = 16, 32, 48 or 64) and the pointers
+ * are aligned for it (locations and their gradient to 16 bytes, weights and theirs to
+ * four elements, the rest as below), three kernels run in turn on `stream`: the record
+ * sort, which leaves every sample's location, weight and query in bucket order (in
+ * grad_sampling_locations, grad_attention_weights and the workspace), the grad_value
+ * owners over those streams, and the location and weight gradients.
+ *
+ * Otherwise the bucket sort keeps its counters and sorted sample indices in the
+ * workspace instead of grad_attention_weights and grad_sampling_locations, so the
+ * location and weight gradient kernel no longer has to run after it: where that kernel
+ * adds nothing into grad_value (the matrix-core owners take every level, overlapping
+ * ones included, and MSDA_GRAD_VALUE_ATOMIC is off) and the call has at least 2^21
+ * samples, the call forks it onto a side stream of the calling thread (created on the
+ * first such call per thread and device, default priority) beside the sort and the
+ * grad_value kernel, and joins the caller's stream at the end of the call (with
+ * MSDA_SOFTMAX, before the grad_value kernel, which then reads the softmax statistics
+ * grad_sample leaves). The fork and join cost the calling thread about 45 us, so smaller
+ * calls, whose GPU time would not hide that, keep one stream.
  * Work before the call on `stream` happens before all of it, and work after the call
  * after all of it, so it stays stream-ordered and can be captured in a HIP graph.
  * The workspace holds 4 bytes per sample, then at least as many bytes as
