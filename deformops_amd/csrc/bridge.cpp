@@ -159,6 +159,11 @@ struct MSDA : torch::autograd::Function<MSDA> {
 Tensor forward(const Tensor& value, const Tensor& shapes, const Tensor& starts, const Tensor& loc, const Tensor& attn,
                bool softmax) {
   const pybind11::gil_scoped_release no_gil;
+  // There is no forward-mode rule. A tangent is refused in every grad mode, as an
+  // autograd.Function without a jvp refuses it: the launch alone would answer without one.
+  for (const Tensor* t : {&value, &loc, &attn})
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->_fw_grad(/*level=*/0).defined(),
+                                "msda: forward-mode differentiation is not supported (an operand has a tangent)");
   const Operands o = normalized(value, shapes, starts, loc, attn);
   if (at::GradMode::is_enabled() && (o.value.requires_grad() || o.loc.requires_grad() || o.attn.requires_grad()))
     return MSDA::apply(o.value, o.shapes, o.starts, o.loc, o.attn, softmax);

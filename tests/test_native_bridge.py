@@ -144,12 +144,25 @@ def test_saved_tensor_hooks_see_the_five_operands(device):
 
 
 @pytest.mark.gpu
-def test_forward_mode_raises_and_no_grad_records_nothing(device):
+@pytest.mark.parametrize("backend", [None, Backend.HIP], ids=["registry", "explicit"])
+@pytest.mark.parametrize("no_grad", [False, True], ids=["grad", "no-grad"])
+@pytest.mark.parametrize("requires_grad", [False, True], ids=["constant", "leaf"])
+@pytest.mark.parametrize("operand", [0, 3, 4], ids=["value", "loc", "weights"])
+def test_a_tangent_is_refused_in_every_grad_mode(device, operand, requires_grad, no_grad, backend):
     args, _ = operands(device)
-    with torch.autograd.forward_ad.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
-        args_dual = [torch.autograd.forward_ad.make_dual(args[0], torch.ones_like(args[0])), *args[1:]]
-        args_dual[0].requires_grad_(True)
-        torch.autograd.forward_ad.unpack_dual(msda(*args_dual))
+    assert msda.get(Backend.HIP) is not None  # the adapter is imported: a registry call tries the bridge first
+    with torch.autograd.forward_ad.dual_level():
+        primal = args[operand].requires_grad_(requires_grad)
+        args[operand] = torch.autograd.forward_ad.make_dual(primal, torch.ones_like(primal))
+        with torch.set_grad_enabled(not no_grad), pytest.raises(NotImplementedError, match="forward-mode"):
+            msda(*args, backend=backend)
+    args[operand] = primal
+    msda(*args, backend=backend)  # outside the level it is an ordinary operand again
+
+
+@pytest.mark.gpu
+def test_no_grad_and_inference_mode_record_nothing(device):
+    args, _ = operands(device)
     args[0].requires_grad_(True)
     with torch.no_grad():
         assert not msda(*args).requires_grad
