@@ -87,12 +87,13 @@ def compile_library(sources: list[Path], target: Path, *, verbose: bool) -> Path
 
 
 def _compile(command: list[str], target: Path, *, verbose: bool) -> Path:
-    """Run ``command -o target``, through a temporary file beside it."""
+    """Run ``command -o target``, through a temporary directory beside it: the linker
+    makes the file itself, so that its mode follows the umask (a file made for it by
+    ``mkstemp`` keeps 0600, and only its owner could load the library)."""
     target.parent.mkdir(parents=True, exist_ok=True)
-    fd, tmp = tempfile.mkstemp(prefix=target.name + ".", suffix=".tmp", dir=target.parent)
-    os.close(fd)
-    cmd = [*command, "-o", tmp]
-    try:
+    with tempfile.TemporaryDirectory(prefix=target.name + ".", suffix=".tmp", dir=target.parent) as folder:
+        built = Path(folder) / target.name
+        cmd = [*command, "-o", str(built)]
         result = subprocess.run(cmd, capture_output=True, text=True, check=False)  # noqa: S603
         if verbose or result.returncode != 0:
             noise = "is not a recognized feature for this target"
@@ -101,10 +102,7 @@ def _compile(command: list[str], target: Path, *, verbose: bool) -> Path:
                 print("\n".join(lines), file=sys.stderr)
         if result.returncode != 0:
             raise subprocess.CalledProcessError(result.returncode, cmd, result.stdout, result.stderr)
-        os.replace(tmp, target)
-    finally:
-        if os.path.exists(tmp):
-            os.unlink(tmp)
+        os.replace(built, target)
     return target
 
 
