@@ -176,6 +176,12 @@ _lock = threading.Lock()
 _loaded: Library | None = None
 
 
+def compile_allowed(compile: bool | str | None) -> bool:  # noqa: A002
+    """Whether a missing library may be built: ``compile``, or ``DEFORMOPS_COMPILE`` for ``None``."""
+    allow = compile if compile is not None else os.environ.get("DEFORMOPS_COMPILE", "0")
+    return str(allow).strip().lower() in {"1", "true", "yes", "on", "always"}
+
+
 def load(*, download: bool | None = None, compile: bool | str | None = None) -> Library:  # noqa: A002, ARG001
     """Load the library once. With ``compile`` truthy a missing library is built first.
 
@@ -196,8 +202,7 @@ def load(*, download: bool | None = None, compile: bool | str | None = None) -> 
             return _loaded
         path = library_path()
         if not path.exists():
-            allow = compile if compile is not None else os.environ.get("DEFORMOPS_COMPILE", "0")
-            if str(allow).strip().lower() in {"1", "true", "yes", "on", "always"}:
+            if compile_allowed(compile):
                 from ... import _build  # noqa: PLC0415
 
                 try:

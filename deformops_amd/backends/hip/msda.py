@@ -46,14 +46,17 @@ def msda_hip(
 def load(*, download: bool | None = None, compile: bool | str | None = None) -> str:  # noqa: A002
     """Load libdeformops_amd.so and its native bridge; return the library's path."""
     path = str(_lib.load(download=download, compile=compile).path)
-    _native.load()
+    _native.load(download=download, compile=compile)
     return path
 
 
 def direct(*tensors: Any, softmax: bool) -> Any:
     """A plain eager GPU call that needs no check the native bridge cannot make, or
-    ``None`` (see ``try_forward`` in csrc/bridge.cpp)."""
-    return _native.load().try_forward(*tensors, softmax)
+    ``None`` (see ``try_forward`` in csrc/bridge.cpp). Also ``None`` until ``load`` has
+    loaded the bridge: which backend a call runs on, and the error of a call that none
+    can run, stay the policy's."""
+    native = _native.loaded()
+    return None if native is None else native.try_forward(*tensors, softmax)
 
 
 if torch.cuda.is_available() and torch.version.hip is not None:
