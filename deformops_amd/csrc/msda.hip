@@ -2626,7 +2626,7 @@ struct MfmaTile {
 //   meta(ref)      its location and weight loads (one K-block ahead),
 //   query(ref)     its query, for the grad_out rows,
 //   weight(ref, m) its attention weight.
-// ncand: how many there are.
+// ncand: how many there are. partial(): whether some may have no corner in the tile.
 
 // Candidates from the counting sort's entries: sample indices, through which location
 // and weight (with softmax the logit and, when kept, the unit's statistics) are gathered.
@@ -2649,6 +2649,7 @@ template <typename T, typename TL, bool SOFTMAX> struct EntrySource {
     SoftStat<float> st;
   };
   __device__ inline Ref ref(uint32_t first) const { return cand_entry(ent, cr, first + uint32_t(lane)); }
+  __device__ static constexpr bool partial() { return false; }
   __device__ inline uint32_t query(Ref e) const { return fdiv(e, div_lp); }
   __device__ inline void meta(Ref e, Meta& d) const {
     const uint32_t q = fdiv(e, div_lp), s = e - q * uint32_t(LP);
@@ -2682,6 +2683,7 @@ template <typename T, typename TL, bool SOFTMAX> struct RecordSource {
   uint32_t pre, n;      // this lane's range: candidates before it, and in it
   uint32_t delta;       // record of its candidate j: j + delta
   uint32_t ncand;
+  int shift;            // RecordLevels::shift
   unsigned char* slots;  // kWave bytes of the wave's LDS
   int lane;
 
@@ -2696,7 +2698,7 @@ template <typename T, typename TL, bool SOFTMAX> struct RecordSource {
 
   // Takes the ranges of the chunks from g on: tile `tile`, in tile row ty, of a level
   // whose first bucket is `kb`.
-  __device__ inline void group(int g, uint32_t kb, int tile, int ntx, int ty, int shift) {
+  __device__ inline void group(int g, uint32_t kb, int tile, int ntx, int ty) {
     g0 = g;
     const int kind = lane / kRecordGroup, c = g + lane - kind * kRecordGroup;
     uint32_t s0 = 0, s1 = 0;
@@ -2752,6 +2754,7 @@ template <typename T, typename TL, bool SOFTMAX> struct RecordSource {
     r.ql = q[r.idx];
     return r;
   }
+  __device__ inline bool partial() const { return shift >= 0; }
   __device__ inline uint32_t query(const Ref& r) const { return r.q0 + r.ql; }
   __device__ inline void meta(const Ref& r, Meta& d) const {
     d.loc = *reinterpret_cast<const LocPair<TL>*>(loc + r.idx * uint32_t(2 * sizeof(TL)));
@@ -2861,8 +2864,8 @@ __device__ inline MfmaCorners mfma_kblock_a(const Source& src, const MfmaTile& t
 
 // TAIL: a tile's last K-blocks, whose second K-step may hold no candidate.
 template <typename T, int NB, int NST, bool TAIL = false>
-__device__ inline void mfma_kblock_b(const MfmaCorners& cr, int lane, const unsigned char* gst, unsigned char* wt,
-                                     f32x4_v (&acc)[4][NB], int ksteps = 2) {
+__device__ inline void mfma_kblock_b(const MfmaCorners& cr, bool partial, int lane, unsigned char* gst,
+                                     unsigned char* wt, f32x4_v (&acc)[4][NB], int ksteps = 2) {
   constexpr bool kSplit = sizeof(T) == 4;
   constexpr bool kF16 = mfma_f16_operands<T>();
   constexpr int kRowBytes = mfma_row_bytes(NB);
@@ -2879,6 +2882,18 @@ __device__ inline void mfma_kblock_b(const MfmaCorners& cr, int lane, const unsi
       for (int k = 0; k < 4; ++k) {
         *reinterpret_cast<uint16_t*>(wt + cr.o[k]) = uint16_t(cr.hi[k / 2] >> (16 * (k & 1)));
         *reinterpret_cast<uint16_t*>(wt + kMfmaLoTiles + cr.o[k]) = uint16_t(cr.lo[k / 2] >> (16 * (k & 1)));
+      }
+      // A candidate without a corner in the tile has zero weights, but its row may hold an
+      // infinity or a NaN that no sample of the tile has (0 x inf is NaN): its lane clears
+      // the staged row.
+      constexpr int kUnroll = !kSplit && NB == 4 ? kRowBytes / 16 : 1;  // rolled, that one spills
+      if (partial && min(min(cr.o[0], cr.o[1]), min(cr.o[2], cr.o[3])) >= uint32_t(kMfmaSpare)) {
+#pragma unroll kUnroll
+        for (int i = 0; i < kRowBytes; i += 16) {
+          *reinterpret_cast<u32x4_v*>(gst + lane * kRowBytes + i) = u32x4_v{0u, 0u, 0u, 0u};
+          if constexpr (kSplit)
+            *reinterpret_cast<u32x4_v*>(gst + kLoRows + lane * kRowBytes + i) = u32x4_v{0u, 0u, 0u, 0u};
+        }
       }
     }
     wave_lds_order();
@@ -2962,12 +2977,12 @@ __device__ inline void mfma_tile_kblocks(const Source& src, const MfmaTile& t, c
     src.meta(eb, mb);
     const auto c0 = mfma_kblock_a<T, NB>(src, t, lv, kb, ea, ma, rows, lane, gst);
     mfma_load_rows<T, NB>(t, src.query(eb), lane, rows);
-    mfma_kblock_b<T, NB, NST>(c0, lane, gst, wt, acc);
+    mfma_kblock_b<T, NB, NST>(c0, src.partial(), lane, gst, wt, acc);
     const typename Source::Ref e3 = src.ref(cand + 3 * step);
     src.meta(e2, ma);
     const auto c1 = mfma_kblock_a<T, NB>(src, t, lv, kb + uint32_t(kbstep), eb, mb, rows, lane, gst);
     mfma_load_rows<T, NB>(t, src.query(e2), lane, rows);
-    mfma_kblock_b<T, NB, NST>(c1, lane, gst, wt, acc);
+    mfma_kblock_b<T, NB, NST>(c1, src.partial(), lane, gst, wt, acc);
     ea = e2;
     eb = e3;
     cand += 2 * step;
@@ -2977,10 +2992,10 @@ __device__ inline void mfma_tile_kblocks(const Source& src, const MfmaTile& t, c
   if (two) src.meta(eb, mb);
   const auto c0 = mfma_kblock_a<T, NB>(src, t, lv, kb, ea, ma, rows, lane, gst);
   if (two) mfma_load_rows<T, NB>(t, src.query(eb), lane, rows);
-  mfma_kblock_b<T, NB, NST, true>(c0, lane, gst, wt, acc, mfma_ksteps(src.ncand, kb));
+  mfma_kblock_b<T, NB, NST, true>(c0, src.partial(), lane, gst, wt, acc, mfma_ksteps(src.ncand, kb));
   if (two) {
     const auto c1 = mfma_kblock_a<T, NB>(src, t, lv, kb + uint32_t(kbstep), eb, mb, rows, lane, gst);
-    mfma_kblock_b<T, NB, NST, true>(c1, lane, gst, wt, acc, mfma_ksteps(src.ncand, kb + uint32_t(kbstep)));
+    mfma_kblock_b<T, NB, NST, true>(c1, src.partial(), lane, gst, wt, acc, mfma_ksteps(src.ncand, kb + uint32_t(kbstep)));
   }
 }
 
@@ -3519,10 +3534,10 @@ msda_record_owner_kernel(const Problem p, const BwdGeom bg, const Records rec, c
   // The task at position k of a list, and its candidate source.
   RecordSource<T, TL, SOFTMAX> src;
   src.row = uint32_t(uni(plan.buckets) + 1);
-  const int shift = uni(plan.shift);
   src.nch = rec.nch;
   src.qc = rec.qc;
   src.LP = LP;
+  src.shift = uni(plan.shift);
   src.slots = wt + kMfmaSpare;
   src.lane = lane;
   auto run = [&](int k, const int* ends, int kb0, int kbstep, f32x4_v (&acc)[4][NB], int& parts) __attribute__((always_inline)) -> Task {
@@ -3566,7 +3581,7 @@ msda_record_owner_kernel(const Problem p, const BwdGeom bg, const Records rec, c
     parts = 0;
     auto groups = [&]<int NST>() __attribute__((always_inline)) {
       for (int g = 0; g < src.nch; g += kRecordGroup) {
-        src.group(g, first_bucket, tile, tl.ntx, ty, shift);
+        src.group(g, first_bucket, tile, tl.ntx, ty);
         parts = max(parts, int((src.ncand + kMfmaK - 1) / kMfmaK));
         mfma_tile_kblocks<T, NB, NST>(src, t, lv, kb0, kbstep, lane, gst, wt, acc);
       }

@@ -59,3 +59,43 @@ def test_record_path_matches_the_oracle_and_the_counting_sort(device, shape, dty
     assert rel_err(got[1], want[1].double().cpu()) <= BWD_TOL[dtype]
     for g, r in zip(got[2:], want[2:]):  # the same kernel on the same inputs
         torch.testing.assert_close(g, r, rtol=0, atol=0)
+
+
+#: levels (all from position 0), batch, queries, heads, positions: one bucket per tile of a
+#: level far from square, one per tile of levels that share positions, one per four tiles
+COARSE = {
+    "line": (((1, 20000),), 1, 20000, 1, 20000),
+    "shared": (((64, 64),) * 8, 48, 640, 8, 4096),
+    "stacked-lines": (((1, 20000),) * 16, 6, 320, 8, 20000),
+}
+
+
+def coarse_operands(shape, dtype, device):
+    """Calls whose owners read coarse buckets: more tiles than the offsets' memory holds."""
+    g = torch.Generator(device).manual_seed(5)
+    levels, B, Q, H, S = COARSE[shape]
+    L, starts = len(levels), (0,) * len(levels)
+    value = torch.randn(B, S, H, 16, generator=g, device=device).to(dtype)
+    loc = torch.rand(B, Q, H, L, 4, 2, generator=g, device=device)
+    attn = torch.rand(B, Q, H, L * 4, generator=g, device=device).to(dtype)
+    grad = torch.randn(B, Q, H * 16, generator=g, device=device).to(dtype)
+    return (value, torch.tensor(levels, device=device), torch.tensor(starts, device=device), loc, attn), grad
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")], ids=["inf", "nan"])
+@pytest.mark.parametrize(("shape", "dtype"), [("line", F32), ("line", BF16), ("shared", BF16), ("stacked-lines", F16)])
+def test_a_nonfinite_channel_reaches_only_the_tiles_its_query_samples(device, shape, dtype, bad):
+    """A product of a zero weight and an infinity is NaN, so a non-finite grad_output channel
+    spoils the whole tile of each of its query's samples, and nothing else: where owners read
+    coarse buckets, the candidates that have no corner in the tile stay out of it."""
+    args, grad = coarse_operands(shape, dtype, device)
+    grad[-1, 7, 3] = bad
+    got = run_hip(*args, grad, softmax=False)[1]
+    with _lib.path_override(_lib.PATH_ATOMIC_SORT):  # the counting sort: a tile's own samples
+        want = run_hip(*args, grad, softmax=False)[1]
+    spoilt = ~torch.isfinite(got)
+    assert spoilt.any() and not (spoilt & torch.isfinite(want)).any()
+    spoilt[-1, :, 0, 3] = False
+    assert not spoilt.any()  # nor any other image, head or channel
+    ok = torch.isfinite(want)
+    assert rel_err(got[ok], want[ok].double().cpu()) <= BWD_TOL[dtype]
