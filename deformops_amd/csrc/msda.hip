@@ -1688,7 +1688,7 @@ __global__ __launch_bounds__(1024) void msda_record_sort_kernel(const Problem p,
   using W = RecordWeight<T, SOFTMAX>;
   using LocWord = std::conditional_t<sizeof(TL) == 2, uint32_t, u32x2_v>;  // one location pair
   __shared__ RecordLevels plan;
-  __shared__ int hist[kRecordKeys];
+  __shared__ __align__(8) int hist[kRecordKeys];
   __shared__ int scan_sums[1024 / kWave];
   extern __shared__ __align__(16) unsigned char stage[];
   const int T_ = int(blockDim.x), tid = int(threadIdx.x);
@@ -1704,11 +1704,16 @@ __global__ __launch_bounds__(1024) void msda_record_sort_kernel(const Problem p,
   const int64_t unit0 = (int64_t(b) * p.Q + q0) * p.H + h;
   const int64_t bh = int64_t(b) * p.H + h;
 
-  // Softmax: a unit's log-sum-exp, formed by one thread per unit first where units are long
-  // (kept where the counters will be: at most 16,384 / 4 units a chunk), else by each of
-  // its L P / 4 groups, which spares the barrier and the idle threads: 42 against 64 us
-  // for 4.7 M samples, 40 a unit, but 72 against 71 us for 8.3 M samples, 12 a unit.
-  auto unit_lse = [&](const T* at) __attribute__((always_inline)) -> float {
+  // Softmax: a unit's largest logit and the logarithm of its sum of exponentials above it,
+  // formed by one thread per unit first where units are long (kept where the counters will
+  // be), else by each of its L P / 4 groups, which spares the barrier and the idle threads:
+  // 42 against 64 us for 4.7 M samples, 40 a unit, but 72 against 71 us for 8.3 M samples,
+  // 12 a unit. The two stay apart: in their sum a logit far from zero, such as a mask's,
+  // swallows the logarithm.
+  struct UnitStat {
+    float mx, ln;
+  };
+  auto unit_stat = [&](const T* at) __attribute__((always_inline)) -> UnitStat {
     float mx = -INFINITY, sum = 0.f;
 #pragma unroll 4
     for (int j = 0; j < LP; j += 4) {
@@ -1723,14 +1728,14 @@ __global__ __launch_bounds__(1024) void msda_record_sort_kernel(const Problem p,
 #pragma unroll
       for (int k = 0; k < 4; ++k) sum += exp_acc(v[k] - mx);
     }
-    return mx + log(sum);
+    return UnitStat{mx, log(sum)};
   };
-  const bool shared_lse = SOFTMAX && LP > kSharedSoftmax;
-  if (shared_lse) {  // uniform
-    static_assert(4 * GP * 1024 / 4 <= kRecordKeys);
+  const bool shared_stat = SOFTMAX && LP > kSharedSoftmax;
+  if (shared_stat) {  // uniform
+    static_assert(4 * GP * 1024 / kSharedSoftmax * 2 <= kRecordKeys);
     if (work)
       for (int q = tid; q < nq; q += T_)
-        reinterpret_cast<float*>(hist)[q] = unit_lse(reinterpret_cast<const T*>(p.attn) + (unit0 + int64_t(q) * p.H) * LP);
+        reinterpret_cast<UnitStat*>(hist)[q] = unit_stat(reinterpret_cast<const T*>(p.attn) + (unit0 + int64_t(q) * p.H) * LP);
     __syncthreads();
   }
 
@@ -1754,9 +1759,9 @@ __global__ __launch_bounds__(1024) void msda_record_sort_kernel(const Problem p,
     if constexpr (SOFTMAX) {
       float a[4];
       Chan<T, 4>::load(reinterpret_cast<const char*>(at + 4 * int(r)), a);
-      const float lse = shared_lse ? reinterpret_cast<const float*>(hist)[q] : unit_lse(at);
+      const UnitStat u = shared_stat ? reinterpret_cast<const UnitStat*>(hist)[q] : unit_stat(at);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) wt[i][k] = exp_acc(a[k] - lse);
+      for (int k = 0; k < 4; ++k) wt[i][k] = exp_acc(a[k] - u.mx - u.ln);
     } else {
       const Raw<4 * sizeof(T)> a = *reinterpret_cast<const Raw<4 * sizeof(T)>*>(at + 4 * int(r));
       __builtin_memcpy(wt[i], &a, sizeof(a));

@@ -99,3 +99,23 @@ def test_a_nonfinite_channel_reaches_only_the_tiles_its_query_samples(device, sh
     assert not spoilt.any()  # nor any other image, head or channel
     ok = torch.isfinite(want)
     assert rel_err(got[ok], want[ok].double().cpu()) <= BWD_TOL[dtype]
+
+
+@pytest.mark.parametrize(("dtype", "offset"), [
+    (F32, -3.4e38), (F32, -1e9), (F32, 1e5), (BF16, -3.38e38), (BF16, -1e9), (F16, -65000.0), (F16, 3e4),
+])
+@pytest.mark.parametrize(("levels", "points", "queries"), [
+    (((24, 24), (12, 12), (6, 6)), 4, 700),  # statistics formed by every group of a unit
+    (((24, 24), (12, 12), (6, 6), (3, 3), (2, 2)), 8, 300),  # by one thread per unit
+], ids=["per-group", "per-unit"])
+def test_softmax_of_logits_far_from_zero(device, levels, points, queries, dtype, offset):
+    """Masks of the type's lowest value, or any offset that swallows the logits: a fully masked
+    unit's weights are 1 / (L P) each, as in the forward. max + log(sum) in one float drops the
+    logarithm beyond about 1e7, and rounds it to 0.008 at 1e5."""
+    w = make_workload(2, batch=2, queries=queries, heads=3, channels=32, points=points, levels=levels,
+                      locations="uniform", seed=4).to(device, dtype, F32)
+    value, shapes, starts, loc, logits = w.operands(softmax=True)
+    logits = logits.clone()
+    logits[:, ::3] = (logits[:, ::3].double() + offset).clamp(torch.finfo(dtype).min, torch.finfo(dtype).max).to(dtype)
+    check_against_oracle(value, shapes, starts, loc, logits, w.grad_output, softmax=True, dtype=dtype,
+                         label=f"offset {offset}")
