@@ -1083,9 +1083,16 @@ __device__ inline bool queue_fits(const Problem& p, const BwdGeom& bg, int64_t n
 // the place pass (over the per-workgroup counts, done with by then), where the
 // scratch has room. A candidate's weight is then exp(logit - lse): one logit and one
 // 4-byte statistics load instead of a pass over the unit's L * P logits.
+// Beyond kStatRange the sum would round the logarithm away (at a mask's -1e9 all of it),
+// so such a unit's statistics are NaN, and its candidates make that pass.
+constexpr float kStatRange = 256.f;  // half a unit in the last place of 256: 1.5e-5 of a float weight
 template <typename A> struct SoftStat {
   A lse;
+  __device__ inline bool ok() const { return lse == lse; }
 };
+template <typename A> __device__ inline SoftStat<A> soft_stat(A mx, A sum) {
+  return SoftStat<A>{fabs(mx) <= A(kStatRange) ? mx + log(sum) : A(NAN)};
+}
 template <typename A>
 __device__ inline SoftStat<A>* softmax_stats(int* buckets, const Problem& p, int64_t nkeys) {
   return reinterpret_cast<SoftStat<A>*>(chunk_counts(buckets, p, nkeys));
@@ -1990,7 +1997,7 @@ __global__ __launch_bounds__(256) void msda_softmax_stats_kernel(const Problem p
       for (int i = 0; i < LP; ++i) mx = fmax(mx, load_acc(lg + i));
       A sum(0);
       for (int i = 0; i < LP; ++i) sum += exp_acc(load_acc(lg + i) - mx);
-      st[u] = SoftStat<A>{mx + log(sum)};
+      st[u] = soft_stat(mx, sum);
     }
     wave_lds_order();  // the lanes' reads come before the next copy
   }
@@ -2332,12 +2339,10 @@ __global__ __launch_bounds__(kOwnerThreads) void msda_grad_value_kernel(
         if constexpr (SOFTMAX) {
           const uint32_t q = fdiv(c_own, bg.div_lp), s = c_own - q * uint32_t(LP);
           const int64_t u = unit0 + int64_t(q) * p.H;
-          if (stats) {
-            const SoftStat<A> st = stats[u];
-            a = exp_acc(load_acc(attn_all + u * LP + s) - st.lse);
-          } else {
-            a = unit_weight<T, true>(attn_all + u * LP, LP, int(s));
-          }
+          SoftStat<A> st{A(NAN)};
+          if (stats) st = stats[u];
+          a = st.ok() ? exp_acc(load_acc(attn_all + u * LP + s) - st.lse)
+                      : unit_weight<T, true>(attn_all + u * LP, LP, int(s));
         } else {
           a = to_acc(c_attn);
         }
@@ -2665,7 +2670,7 @@ template <typename T, typename TL, bool SOFTMAX> struct EntrySource {
   }
   __device__ inline float weight(Ref e, const Meta& d) const {
     if constexpr (SOFTMAX) {
-      if (stats) return exp_acc(to_acc(d.attn) - d.st.lse);
+      if (stats && d.st.ok()) return exp_acc(to_acc(d.attn) - d.st.lse);
       const uint32_t q = fdiv(e, div_lp), s = e - q * uint32_t(LP);
       return unit_weight<T, true>(reinterpret_cast<const T*>(attn + __umul24(q, attn_q)), LP, int(s));
     } else {
@@ -3754,7 +3759,7 @@ __global__ __launch_bounds__(kWave * kMaxWavesPerBlock) void msda_grad_sample_ke
   A smax, sinv, ssum = A(1);
   unit_softmax<T, SOFTMAX>(m, LP, raw, smax, sinv, &ssum);
   if constexpr (SOFTMAX)  // the unit's log-sum-exp for the grad_value kernel, as msda_softmax_stats_kernel's
-    if (p.stats && m.unit_ok && m.t == 0) reinterpret_cast<SoftStat<A>*>(p.stats)[m.gunit] = SoftStat<A>{smax + log(ssum)};
+    if (p.stats && m.unit_ok && m.t == 0) reinterpret_cast<SoftStat<A>*>(p.stats)[m.gunit] = soft_stat(smax, ssum);
   __syncthreads();
   // grad_value by atomics: asked for, or levels overlap where the owners stand aside
   // (the sort and the owners then only zeroed grad_value).

@@ -107,7 +107,8 @@ def test_a_nonfinite_channel_reaches_only_the_tiles_its_query_samples(device, sh
 @pytest.mark.parametrize(("levels", "points", "queries"), [
     (((24, 24), (12, 12), (6, 6)), 4, 700),  # statistics formed by every group of a unit
     (((24, 24), (12, 12), (6, 6), (3, 3), (2, 2)), 8, 300),  # by one thread per unit
-], ids=["per-group", "per-unit"])
+    (((24, 24), (12, 12), (6, 6)), 3, 700),  # the counting sort's, where they fit their range
+], ids=["per-group", "per-unit", "counting-sort"])
 def test_softmax_of_logits_far_from_zero(device, levels, points, queries, dtype, offset):
     """Masks of the type's lowest value, or any offset that swallows the logits: a fully masked
     unit's weights are 1 / (L P) each, as in the forward. max + log(sum) in one float drops the
