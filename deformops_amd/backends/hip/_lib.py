@@ -66,6 +66,7 @@ EXPORTED_SYMBOLS = (
     "msda_last_error",
     "msda_abi_version",
     "msda_launch_geometry",
+    "msda_record_plan",
     "msda_set_path_override",
     "msda_set_phase_events",
 )
@@ -170,6 +171,17 @@ class Library:
             "waves_per_block": waves.value,
             "num_blocks": blocks.value,
         }
+
+    def record_plan(self, dtype: torch.dtype, loc_dtype: torch.dtype, sizes: tuple[int, ...],
+                    flags: int = 0) -> tuple[int, int, int]:
+        """``(queries per chunk, chunks per (image, head), bucket offsets that fit)`` of the
+        record sort for a workspace call of sizes ``(B, S, H, D, Q, L, P)``, all 0 where
+        the counting sort takes it (host only)."""
+        queries, chunks, offsets = _I(), _I(), _L()
+        self.check(self.cdll.msda_record_plan(
+            DTYPE_CODES[dtype], DTYPE_CODES[loc_dtype], *(_L(n) for n in sizes), flags,
+            ctypes.byref(queries), ctypes.byref(chunks), ctypes.byref(offsets)))
+        return queries.value, chunks.value, offsets.value
 
 
 _lock = threading.Lock()

@@ -886,7 +886,8 @@ struct Records {
   char* w;         // attention weights: RecordWeight
   uint16_t* q;     // query - c qc
   uint16_t* offs;  // per (b, h, chunk): the first record of every bucket, then the end
-  int* queue;      // the matrix-core kernel's kXcds work-queue counters, one per 128-byte line
+  int* queue;      // the owners' work queues: per XCD a 128-byte line with the next split task,
+                   // then the next whole task (zeroed by the sort)
   int64_t offs_cap;  // entries the offsets' memory holds
   int qc, nch;     // queries per chunk, chunks per (b, h)
 };
@@ -4384,6 +4385,20 @@ RecordPlan make_record_plan(int64_t B, int64_t S, int64_t H, int64_t Q, int64_t 
   return r;
 }
 
+// The record path's chunks for a call whose pointers are aligned for it, with `counters`
+// bytes of workspace for the owners' work queues and the bucket offsets (16 bits each;
+// offs_cap: how many). Not ok: the counting sort takes the call.
+constexpr int64_t kRecordQueueBytes = int64_t(kXcds) * kQueueLine * 4;
+RecordPlan record_plan_of(const BackwardPlan& plan, int64_t B, int64_t S, int64_t H, int64_t Q, int64_t L, int64_t P,
+                          int flags, int paths, int64_t counters, int64_t* offs_cap) {
+  const int64_t most = flags & MSDA_SOFTMAX ? kRecordSoftmaxSamples : kRecordSamples;
+  *offs_cap = (counters - kRecordQueueBytes) / 2;
+  if (!plan.mfma || plan.mfma_fallback || (flags & MSDA_GRAD_VALUE_ATOMIC) || (paths & MSDA_PATH_ATOMIC_SORT) ||
+      L > kRecordLevels || P % 4 != 0 || L * P > most || S >= kRecordPositions)
+    return RecordPlan{};
+  return make_record_plan(B, S, H, Q, L, P, plan.bg.small_tiles, *offs_cap);
+}
+
 template <typename T, typename TL, bool SM>
 hipError_t launch_record_sort(const BackwardPlan& plan, const RecordPlan& rp, const Problem& p, const Records& rec,
                               hipStream_t st) {
@@ -4726,6 +4741,33 @@ int msda_launch_geometry(int value_dtype, int64_t batch, int64_t spatial, int64_
   return MSDA_OK;
 }
 
+int msda_record_plan(int value_dtype, int loc_dtype, int64_t batch, int64_t spatial, int64_t heads, int64_t channels,
+                     int64_t queries, int64_t levels, int64_t points, int flags, int* chunk_queries, int* chunks,
+                     int64_t* offsets) {
+  g_last_error[0] = '\0';
+  const int rc = check_call(value_dtype, MSDA_I64, loc_dtype, batch, spatial, heads, channels, queries, levels, points,
+                            flags, MSDA_SOFTMAX | MSDA_ACCUMULATE_GRAD_VALUE | MSDA_GRAD_VALUE_ATOMIC);
+  if (rc != MSDA_OK) return rc;
+  RecordPlan rp = {};
+  int64_t cap = 0;
+  if (batch * queries * heads * levels * points > 0 && channels > 0 && spatial > 0) {
+    const bool softmax = flags & MSDA_SOFTMAX;
+    const WorkspaceLayout wl = workspace_layout(value_dtype, batch, spatial, heads, queries, levels, points, softmax);
+    const int paths = g_path_override.load(std::memory_order_relaxed);
+    BackwardPlan plan;
+    const int rc2 = make_backward_plan(value_dtype, batch, spatial, heads, channels, queries, levels, points, loc_dtype,
+                                       nullptr, 0, nullptr, 160 * 1024, 256, &plan, flags & MSDA_ACCUMULATE_GRAD_VALUE,
+                                       paths, wl.counters_bytes);
+    if (rc2 != MSDA_OK) return rc2;
+    rp = record_plan_of(plan, batch, spatial, heads, queries, levels, points, flags, paths, wl.total - wl.counters_off,
+                        &cap);
+  }
+  if (chunk_queries) *chunk_queries = rp.ok ? rp.qc : 0;
+  if (chunks) *chunks = rp.ok ? rp.nch : 0;
+  if (offsets) *offsets = rp.ok ? cap : 0;
+  return MSDA_OK;
+}
+
 int msda_forward(const void* value, int value_dtype, const void* spatial_shapes,
                  const void* level_start_index, int index_dtype, const void* sampling_locations,
                  int loc_dtype, const void* attention_weights, void* output, int64_t batch,
@@ -4867,20 +4909,18 @@ static int backward_call(const void* value, int value_dtype, const void* spatial
   // float: those take the index region and the query numbers grad_attention_weights.
   Records rec = {};
   RecordPlan rp = {};
-  if (use_ws && plan.mfma && !plan.mfma_fallback && !atomic_gv && levels <= kRecordLevels && points % 4 == 0 &&
-      levels * points <= (softmax ? kRecordSoftmaxSamples : kRecordSamples) && spatial < kRecordPositions &&
-      aligned(sampling_locations, 16) && aligned(attention_weights, 4 * es) && aligned(grad_sampling_locations, 16) &&
-      aligned(grad_attention_weights, 4 * es) && !(paths & MSDA_PATH_ATOMIC_SORT)) {
-    const int64_t queue_bytes = int64_t(kXcds) * kQueueLine * 4;
-    const int64_t cap = (workspace_bytes - wl.counters_off - queue_bytes) / 2;
-    rp = make_record_plan(batch, spatial, heads, queries, levels, points, plan.bg.small_tiles, cap);
+  if (use_ws && aligned(sampling_locations, 16) && aligned(attention_weights, 4 * es) &&
+      aligned(grad_sampling_locations, 16) && aligned(grad_attention_weights, 4 * es)) {
+    int64_t cap = 0;
+    rp = record_plan_of(plan, batch, spatial, heads, queries, levels, points, flags, paths,
+                        workspace_bytes - wl.counters_off, &cap);
     if (rp.ok) {
       const bool wide = softmax && es == 2;  // 4-byte weights of 16-bit logits
       rec.loc = static_cast<char*>(grad_sampling_locations);
       rec.w = static_cast<char*>(wide ? workspace : grad_attention_weights);
       rec.q = static_cast<uint16_t*>(wide ? grad_attention_weights : workspace);
       rec.queue = static_cast<int*>(counters);
-      rec.offs = reinterpret_cast<uint16_t*>(static_cast<char*>(counters) + queue_bytes);
+      rec.offs = reinterpret_cast<uint16_t*>(static_cast<char*>(counters) + kRecordQueueBytes);
       rec.offs_cap = cap;
       rec.qc = rp.qc;
       rec.nch = rp.nch;

@@ -156,10 +156,13 @@ int msda_backward(const void* value, int value_dtype,
  * bytes for the same sizes (device memory, 256-byte aligned; its contents are
  * ignored and left undefined). Writes the same three gradients.
  *
- * Where P is a multiple of 4, L at most 16, an image under 2^20 positions, the matrix
- * cores take grad_value (16-bit or float values, D = 16, 32, 48 or 64) and the pointers
- * are aligned for it (locations and their gradient to 16 bytes, weights and theirs to
- * four elements, the rest as below), three kernels run in turn on `stream`: the record
+ * Where P is a multiple of 4, L at most 16, L * P at most 1,024 (64 with MSDA_SOFTMAX),
+ * an image under 2^20 positions, MSDA_GRAD_VALUE_ATOMIC off, the matrix cores take
+ * grad_value (16-bit or float values, D = 16, 32, 48 or 64), the pointers are aligned for
+ * it (locations and their gradient to 16 bytes, weights and theirs to four elements, the
+ * rest as below) and the workspace holds the sort's bucket offsets (a workspace of
+ * msda_backward_workspace_size bytes does, but for few samples against many positions;
+ * msda_record_plan tells), three kernels run in turn on `stream`: the record
  * sort, which leaves every sample's location, weight and query in bucket order (in
  * grad_sampling_locations, grad_attention_weights and the workspace), the grad_value
  * owners over those streams, and the location and weight gradients.
@@ -266,6 +269,19 @@ int msda_launch_geometry(int value_dtype, int64_t batch, int64_t spatial,
                          int64_t levels, int64_t points, int backward,
                          int* channels_per_lane, int* lanes_per_unit,
                          int* waves_per_block, int64_t* num_blocks);
+
+/* How msda_backward_workspace sorts the samples of a call of these sizes, dtypes and
+ * flags with a workspace of msda_backward_workspace_size bytes and aligned pointers: the
+ * queries of one chunk of the record sort, the chunks of one (image, head), and how many
+ * 16-bit bucket offsets the workspace holds; all 0 where the counting sort takes the
+ * call. (A chunk has 4 offsets per tile and one more; where batch * heads * chunks of
+ * those do not fit, the kernels take one bucket per two, four, ... tiles of a level.)
+ * Host only; lets a test see which path its sizes take. No counterpart in the
+ * reference. */
+int msda_record_plan(int value_dtype, int loc_dtype, int64_t batch, int64_t spatial,
+                     int64_t heads, int64_t channels, int64_t queries, int64_t levels,
+                     int64_t points, int flags, int* chunk_queries, int* chunks,
+                     int64_t* offsets);
 
 #ifdef __cplusplus
 }

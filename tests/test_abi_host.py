@@ -207,6 +207,51 @@ def test_launch_geometry_takes_as_many_samples_as_fit_one_wave_whole(lib, dtype,
         assert rc == (0 if fits(samples) else 2), samples
 
 
+def test_every_row_of_the_record_tests_takes_the_path_it_stands_for(lib):
+    """Sizes of tests/test_hip_records.py: a row the counting sort took would compare that
+    with itself."""
+    from tests.test_hip_records import COARSE, DTYPES, SHAPES, record_chunks  # noqa: PLC0415
+
+    for name, (levels, B, Q, H, D, P) in SHAPES.items():  # noqa: N806
+        sizes = (B, sum(h * w for h, w in levels), H, D, Q, len(levels), P)
+        for dtype, loc_dtype in DTYPES:
+            for softmax in (False, True):
+                chunk, chunks, shift = record_chunks(levels, sizes, dtype, loc_dtype, softmax=softmax)
+                assert chunk > 0 and (chunks - 1) * chunk < Q <= chunks * chunk, (name, dtype, softmax)
+                if not (name == "line" and softmax):
+                    assert (shift >= 0) == (name == "line"), (name, dtype, softmax)
+                assert (chunks > 21) == (name == "many-chunks"), (name, dtype, softmax)
+                if name == "long-units":  # more than 16 samples a unit, and than one group a thread
+                    assert len(levels) * P > 16 and chunk * len(levels) * P > 4096
+    for name, shift in {"line": 0, "shared": 0, "stacked-lines": 2}.items():
+        levels, B, Q, H, S = COARSE[name]  # noqa: N806
+        sizes = (B, S, H, 16, Q, len(levels), 4)
+        dtype = {"line": torch.bfloat16, "shared": torch.bfloat16, "stacked-lines": torch.float16}[name]
+        assert record_chunks(levels, sizes, dtype, torch.float32)[2] == shift, name
+
+
+def test_the_record_plan_says_which_calls_the_counting_sort_takes(lib):
+    sizes = (2, 5376, 8, 32, 5376, 3, 4)
+    bf16, f32, f64 = torch.bfloat16, torch.float32, torch.float64
+    assert lib.record_plan(bf16, f32, sizes)[0] > 0
+    taken = {
+        "points": lib.record_plan(bf16, f32, (*sizes[:6], 3)),
+        "dtype": lib.record_plan(f64, f64, sizes),
+        "channels": lib.record_plan(bf16, f32, (2, 5376, 8, 40, 5376, 3, 4)),
+        "atomics": lib.record_plan(bf16, f32, sizes, _lib.FLAG_GRAD_VALUE_ATOMIC),
+        "levels": lib.record_plan(bf16, f32, (2, 5376, 8, 32, 100, 17, 4)),
+        "softmax samples": lib.record_plan(bf16, f32, (2, 5376, 8, 32, 100, 5, 16), _lib.FLAG_SOFTMAX),
+        "positions": lib.record_plan(bf16, f32, (1, 1 << 20, 1, 32, 100, 1, 4)),
+        "empty": lib.record_plan(bf16, f32, (2, 5376, 8, 32, 0, 3, 4)),
+    }
+    assert all(plan == (0, 0, 0) for plan in taken.values()), taken
+    assert lib.record_plan(bf16, f32, (2, 5376, 8, 32, 100, 5, 16))[0] > 0  # linear: up to 1,024 samples
+    with _lib.path_override(_lib.PATH_ATOMIC_SORT):
+        assert lib.record_plan(bf16, f32, sizes) == (0, 0, 0)
+    with pytest.raises(RuntimeError, match="locations"):
+        lib.record_plan(bf16, torch.float16, sizes)
+
+
 @pytest.mark.parametrize(
     ("levels", "points", "dtype", "head_dim", "expected"),
     [

@@ -4,7 +4,9 @@ path, at the sizes where they can go wrong: chunks that are exactly full, one sa
 short or a single query; more chunks than one wave holds ranges of; more buckets than
 the LDS counters; tables whose bucket offsets need coarse buckets; tile and level
 edges; heads of 16 to 64 channels; levels long and short enough for split and for
-per-wave tasks.
+per-wave tasks; units of more samples than share a softmax, in chunks of one and of four
+groups a thread. tests/test_abi_host.py checks that every row takes the path it stands
+for.
 
 Tolerances are the parity suite's: float32 1e-4 (grad_value's products of split 16-bit
 parts have relative error at most 3 * 2^-16 = 4.6e-5 each), 16-bit 2e-2 of the largest
@@ -32,13 +34,33 @@ SHAPES = {
     "many-chunks": (((33, 31),), 1, 90001, 1, 16, 4),
     "many-buckets": (((400, 400), (9, 9)), 1, 3000, 1, 16, 4),
     "line": (((1, 20000),), 1, 20000, 1, 16, 4),
-    "lines": (((3, 7000), (9000, 1)), 1, 9000, 1, 16, 4),
+    "lines": (((3, 7000), (9000, 1)), 1, 20000, 1, 16, 4),
     "tile-edges": (((7, 9), (8, 8), (9, 17), (1, 1), (24, 16)), 2, 1003, 3, 48, 4),
     "wide-heads": (((19, 25), (10, 13)), 1, 4001, 2, 64, 8),
     "decoder": (((100, 134), (50, 67), (25, 34), (13, 17)), 2, 301, 4, 32, 4),
     "coarse-and-fine": (((64, 64), (4, 4)), 2, 5000, 4, 32, 4),
+    "long-units": (((40, 50), (20, 25), (10, 13), (5, 7), (3, 4)), 1, 5000, 2, 32, 4),
 }
 DTYPES = [(F32, F32), (BF16, BF16), (F16, F16), (BF16, F32), (F16, F32)]
+
+
+def record_chunks(levels, sizes, dtype, loc_dtype, *, softmax=False):
+    """``(queries per chunk, chunks per (image, head), log2 of the tiles per bucket)`` of a
+    call's record sort, the last -1 where a tile has four buckets of its own; 0 chunks
+    where the counting sort takes the call (host only)."""
+    B, _, H, _, Q, L, P = sizes
+    chunk, chunks, offsets = _lib.load().record_plan(dtype, loc_dtype, sizes, _lib.FLAG_SOFTMAX if softmax else 0)
+    tiles = 0
+    for h, w in levels:
+        t8 = -(-h // 8) * -(-w // 8)
+        side = 4 if B * H * t8 < 384 and 13 * Q * P >= 24 * 640 * t8 else 8
+        tiles += -(-h // side) * -(-w // side)
+    if B * H * chunks * (4 * tiles + 1) <= offsets:
+        return chunk, chunks, -1
+    shift = 0
+    while B * H * chunks * ((tiles >> shift) + L + 1) > offsets:
+        shift += 1
+    return chunk, chunks, shift
 
 
 @pytest.mark.parametrize("softmax", [False, True], ids=["linear", "softmax"])
