@@ -152,8 +152,8 @@ def settle_clocks(w, softmax: bool, seconds: float = SETTLE_S) -> dict[str, floa
 
 def time_calls(w, steps: int, warmup: int, softmax: bool, bwd_flags: int) -> dict[str, float]:
     """Average device time of the C-ABI calls on torch's current stream: the forward
-    (one kernel), the backward (the bucket sort, the softmax statistics, grad_value,
-    grad_sample), and a forward then a backward back to back."""
+    (one kernel), the backward (the sort, grad_value, grad_sample), and a forward then a
+    backward back to back."""
     from deformops_amd.backends.hip import _lib  # noqa: PLC0415
 
     lib = _lib.load()
@@ -449,7 +449,7 @@ def main() -> int:
         # forward call, and the backward's grad_value and grad_sample phases), and the
         # probe's profiled count over its live launch time (from its GB/s).
         peak = requests["probe_l2"] / (PROBE_BYTES / (gather["l2"] * 1e9)) / 1e9
-        live = {"msda_forward_kernel": calls["forward"], "msda_grad_value_mfma_kernel": calls["phase_grad_value"],
+        live = {"msda_forward_kernel": calls["forward"], "msda_record_owner_kernel": calls["phase_grad_value"],
                 "msda_grad_sample_kernel": calls["phase_grad_sample"]}
         kernels = {}
         for kernel, ms in live.items():
@@ -499,8 +499,8 @@ def main() -> int:
         "roofline": {
             # The contract's roofline is HBM bandwidth (the op is a gather / scatter:
             # no MFMA-bound formulation). The limit the kernels meet below it is the L2
-            # request rate of their row gathers (forward, grad_sample) and the latency
-            # of grad_value's scattered candidate reads: "binding" and "l2_requests".
+            # request rate of their row gathers (forward, grad_sample) and the LDS and the
+            # serial chain of a block of candidates (grad_value): "binding", "l2_requests".
             "bound": "hbm",
             "binding": "l2_request_rate (forward, grad_sample); lds (grad_value)",
             "kernel": "one msda_forward + msda_backward_workspace C-ABI call pair (forward kernel, record sort, "

@@ -24,7 +24,7 @@ from tests.workloads import make_workload
 
 pytestmark = pytest.mark.gpu
 
-F32, BF16, F16 = torch.float32, torch.bfloat16, torch.float16
+F32, BF16, F16, F64 = torch.float32, torch.bfloat16, torch.float16, torch.float64
 
 #: levels, batch, queries, heads, channels, points
 SHAPES = {
@@ -125,6 +125,7 @@ def test_a_nonfinite_channel_reaches_only_the_tiles_its_query_samples(device, sh
 
 @pytest.mark.parametrize(("dtype", "offset"), [
     (F32, -3.4e38), (F32, -1e9), (F32, 1e5), (BF16, -3.38e38), (BF16, -1e9), (F16, -65000.0), (F16, 3e4),
+    (F64, -1e9),  # the counting sort and the owner kernel on vector units
 ])
 @pytest.mark.parametrize(("levels", "points", "queries"), [
     (((24, 24), (12, 12), (6, 6)), 4, 700),  # statistics formed by every group of a unit
@@ -136,7 +137,7 @@ def test_softmax_of_logits_far_from_zero(device, levels, points, queries, dtype,
     unit's weights are 1 / (L P) each, as in the forward. max + log(sum) in one float drops the
     logarithm beyond about 1e7, and rounds it to 0.008 at 1e5."""
     w = make_workload(2, batch=2, queries=queries, heads=3, channels=32, points=points, levels=levels,
-                      locations="uniform", seed=4).to(device, dtype, F32)
+                      locations="uniform", seed=4).to(device, dtype, F64 if dtype is F64 else F32)
     value, shapes, starts, loc, logits = w.operands(softmax=True)
     logits = logits.clone()
     logits[:, ::3] = (logits[:, ::3].double() + offset).clamp(torch.finfo(dtype).min, torch.finfo(dtype).max).to(dtype)
