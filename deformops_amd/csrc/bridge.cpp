@@ -128,6 +128,22 @@ variable_list launch_backward(const Operands& o, const Tensor& grad_output, bool
   return {grad_value, grad_loc, grad_attn};
 }
 
+// Whether the five operands are plain memory of one GPU and agree in rank and size: the
+// launches take addresses and sizes at their word.
+bool agree(const std::array<Tensor, 5>& t) {
+  const Tensor &value = t[0], &shapes = t[1], &starts = t[2], &loc = t[3], &attn = t[4];
+  for (const Tensor& x : t)
+    if (!x.is_cuda() || x.device() != value.device() || x.layout() != at::kStrided) return false;
+  if (value.dim() != 4 || shapes.dim() != 2 || starts.dim() != 1 || loc.dim() != 6) return false;
+  const int64_t B = value.size(0), H = value.size(2), L = shapes.size(0), Q = loc.size(1), P = loc.size(4);
+  if (shapes.size(1) != 2 || starts.size(0) != L || loc.size(0) != B || loc.size(2) != H || loc.size(3) != L ||
+      loc.size(5) != 2)
+    return false;
+  const bool flat = attn.dim() == 4 && attn.size(3) == L * P;
+  const bool split = attn.dim() == 5 && attn.size(3) == L && attn.size(4) == P;
+  return (flat || split) && attn.size(0) == B && attn.size(1) == Q && attn.size(2) == H;
+}
+
 struct MSDA : torch::autograd::Function<MSDA> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& value, const Tensor& shapes,
                         const Tensor& starts, const Tensor& loc, const Tensor& attn, bool softmax) {
@@ -141,8 +157,14 @@ struct MSDA : torch::autograd::Function<MSDA> {
     variable_list out;
     {
       const at::NoGradGuard no_grad;
-      out = launch_backward(Operands{saved[0], saved[1], saved[2], saved[3], saved[4]}, grads[0],
-                            ctx->saved_data["softmax"].toBool());
+      // Saved-tensor hooks may hand back other tensors than they were given: any layout
+      // will do, but not host memory or other sizes.
+      const std::array<Tensor, 5> t = {saved[0], saved[1], saved[2], saved[3], saved[4]};
+      TORCH_CHECK(agree(t) && grads[0].device() == t[0].device() &&
+                      grads[0].sizes() == at::IntArrayRef({t[0].size(0), t[3].size(1), t[0].size(2) * t[0].size(3)}),
+                  "msda: the operands unpacked for the backward are not on the output's device or not of the sizes "
+                  "that were saved");
+      out = launch_backward(normalized(t[0], t[1], t[2], t[3], t[4]), grads[0], ctx->saved_data["softmax"].toBool());
     }
     // The kernels' gradients carry no graph: where one is asked for and would lead
     // through the output's gradient, they come back behind a node that raises.
@@ -185,17 +207,9 @@ bool takes(const std::array<Tensor, 5>& t) {
                                          c10::DispatchKey::BatchedNestedTensor, c10::DispatchKey::Functionalize,
                                          c10::DispatchKey::Python, c10::DispatchKey::Negative});
   for (const Tensor& x : t)
-    if (!x.is_cuda() || x.device() != value.device() || x.layout() != at::kStrided || x.key_set().has_any(wrapped))
-      return false;
-  if (value.dim() != 4 || shapes.dim() != 2 || starts.dim() != 1 || loc.dim() != 6) return false;
-  const int64_t B = value.size(0), S = value.size(1), H = value.size(2), D = value.size(3);
-  const int64_t L = shapes.size(0), Q = loc.size(1), P = loc.size(4), samples = L * P;
-  if (shapes.size(1) != 2 || starts.size(0) != L || loc.size(0) != B || loc.size(2) != H || loc.size(3) != L ||
-      loc.size(5) != 2)
-    return false;
-  const bool flat = attn.dim() == 4 && attn.size(3) == samples;
-  const bool split = attn.dim() == 5 && attn.size(3) == L && attn.size(4) == P;
-  if (!(flat || split) || attn.size(0) != B || attn.size(1) != Q || attn.size(2) != H) return false;
+    if (x.key_set().has_any(wrapped)) return false;
+  if (!agree(t)) return false;
+  const int64_t S = value.size(1), H = value.size(2), D = value.size(3), L = shapes.size(0), samples = L * loc.size(4);
   const at::ScalarType dtype = value.scalar_type(), loc_dtype = loc.scalar_type();
   const bool f64 = dtype == at::kDouble;
   auto kernel_dtype = [](at::ScalarType d) {

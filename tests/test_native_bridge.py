@@ -144,6 +144,36 @@ def test_saved_tensor_hooks_see_the_five_operands(device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name", ["value", "loc", "attn"])
+@pytest.mark.parametrize("change", ["host", "sizes", "strided"])
+def test_unpacked_operands_of_another_kind(device, change, name):
+    """A saved-tensor hook that hands back host memory or other sizes is an error before the
+    launch; other strides are read as what they hold."""
+    (value, shapes, starts, loc, attn), grad = operands(device)
+    leaves = [t.clone().requires_grad_(True) for t in (value, loc, attn)]
+    target = {"value": value, "loc": loc, "attn": attn}[name]
+
+    def unpack(t):  # noqa: ANN001, ANN202
+        if t.shape != target.shape:
+            return t
+        if change == "host":
+            return t.cpu()
+        return t[:, :, :1] if change == "sizes" else t.transpose(1, 2).contiguous().transpose(1, 2)
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        out = msda(leaves[0], shapes, starts, *leaves[1:])
+    if change != "strided":
+        with pytest.raises(RuntimeError, match="unpacked for the backward"):
+            out.backward(grad)
+        return
+    got = torch.autograd.grad(out, leaves, grad)
+    want = torch.autograd.grad(msda(leaves[0], shapes, starts, *leaves[1:]), leaves, grad)
+    torch.testing.assert_close(got[0], want[0], rtol=1e-5, atol=1e-5)
+    for a, b in zip(got[1:], want[1:]):
+        torch.testing.assert_close(a, b, rtol=0, atol=0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("backend", [None, Backend.HIP], ids=["registry", "explicit"])
 @pytest.mark.parametrize("no_grad", [False, True], ids=["grad", "no-grad"])
 @pytest.mark.parametrize("requires_grad", [False, True], ids=["constant", "leaf"])
