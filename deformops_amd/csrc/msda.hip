@@ -916,7 +916,7 @@ __device__ inline int log2_ceil(int v) {
 
 // Tiles of one level. Tile sides are powers of two, so that tiles and sub-buckets
 // follow from shifts and masks; a tile may reach past the level's right or bottom
-// edge. `base` is left to number_tiles.
+// edge. `base` is left to the caller.
 __device__ inline LevelTiles level_tiles(const Problem& p, const BwdGeom& bg, const Level& lv) {
   LevelTiles t{0, 0, 0, 0, 0};
   if (lv.ok && bg.sub_log2 > 0) {
@@ -952,18 +952,6 @@ __device__ inline LevelTiles level_tiles(const Problem& p, const BwdGeom& bg, co
     t.nty = (lv.h + th - 1) >> t.lh;
   }
   return t;
-}
-
-// Numbers the levels' tiles one after the other (one thread). Returns the tile count
-// of one (b, h), or -1 when it exceeds 2^29.
-__device__ inline int64_t number_tiles(int L, LevelTiles* lt) {
-  int64_t total = 0;
-  for (int l = 0; l < L; ++l) {
-    lt[l].base = int(total);
-    total += int64_t(lt[l].ntx) * lt[l].nty;
-    if (total > (int64_t(1) << 29)) return -1;
-  }
-  return total;
 }
 
 // The bucket key of an in-range sample at level l: 4 * tile + sub-bucket.
@@ -1032,6 +1020,17 @@ __device__ inline typename Elem<T>::acc unit_weight(const T* unit_attn, int LP, 
   }
 }
 
+// Whether lane l's level shares positions of S with another lane's (valid ones; L of them).
+__device__ inline bool wave_levels_overlap(int L, int l, const Level& lv) {
+  const int a0 = lv.start, a1 = lv.start + lv.h * lv.w;
+  bool any = false;
+  for (int j = 0; j < L; ++j) {
+    const int b0 = __builtin_amdgcn_readlane(a0, j), b1 = __builtin_amdgcn_readlane(a1, j);
+    any = any || (j != l && lv.ok && __builtin_amdgcn_readlane(lv.ok, j) && a0 < b1 && b0 < a1);
+  }
+  return any;
+}
+
 // Shared set-up of the bucketing kernels and the owners: the level table and the
 // tiles in LDS. Returns the tile count of one (b, h), or -1 when there are too many
 // tiles. When valid levels overlap (`overlap` then says so), the matrix-core owners
@@ -1040,14 +1039,38 @@ __device__ inline typename Elem<T>::acc unit_weight(const T* unit_attn, int LP, 
 // with atomics.
 __device__ inline int64_t load_tiles(const Problem& p, const BwdGeom& bg, Level* levels,
                                      LevelTiles* lt, int64_t* total_out, bool* overlap = nullptr) {
-  if (threadIdx.x == 0) *overlap_flag() = 0;
-  load_levels(p, levels);
+  // By the first wave, a lane for each of 64 levels, in registers, with one barrier: the
+  // backward of B = 4, 300 queries, D = 24, four levels of three points takes 62 us, 65 with
+  // the tiles numbered by one thread behind two barriers more.
+  const int lane = int(threadIdx.x);
+  if (lane < kWave) {
+    int64_t total = 0;
+    bool any = false;
+    for (int l0 = 0; l0 < p.L; l0 += kWave) {
+      const int l = l0 + lane;
+      const Level lv = l < p.L ? load_level(p, l) : Level{1, 1, 0, 0};
+      LevelTiles t = level_tiles(p, bg, lv);
+      const int n = t.ntx * t.nty;  // at most S; summed in two halves, L S may exceed 2^31
+      const int hi = wave_inclusive_scan(n >> 16), lo = wave_inclusive_scan(n & 0xffff);
+      t.base = int(total + (int64_t(hi) << 16) + lo - n);
+      total += (int64_t(__builtin_amdgcn_readlane(hi, kWave - 1)) << 16) + __builtin_amdgcn_readlane(lo, kWave - 1);
+      if (p.L <= kWave) any = wave_levels_overlap(p.L, l, lv);
+      if (l < p.L) {
+        levels[l] = lv;
+        lt[l] = t;
+      }
+    }
+    any = __any(any);
+    if (lane == 0) {
+      *overlap_flag() = any;
+      *total_out = total <= (int64_t(1) << 29) ? total : -1;
+    }
+  }
   __syncthreads();
-  overlap_flag_raise(levels, p.L);
-  for (int l = threadIdx.x; l < p.L; l += blockDim.x) lt[l] = level_tiles(p, bg, levels[l]);
-  __syncthreads();
-  if (threadIdx.x == 0) *total_out = number_tiles(p.L, lt);
-  __syncthreads();
+  if (p.L > kWave) {
+    overlap_flag_raise(levels, p.L);
+    __syncthreads();
+  }
   const bool any = *overlap_flag() != 0;
   if (overlap) *overlap = any;
   return any && !p.sort_overlap ? -1 : *total_out;
@@ -1658,12 +1681,7 @@ __device__ inline RecordLevels& plan_records(const Problem& p, const BwdGeom& bg
   const Level lv = mine ? load_level(p, l) : Level{1, 1, 0, 0};
   LevelTiles t = level_tiles(p, bg, lv);
   const int nt = t.ntx * t.nty;
-  const int a0 = lv.start, a1 = lv.start + lv.h * lv.w;
-  bool any = false;
-  for (int j = 0; j < p.L; ++j) {
-    const int b0 = __builtin_amdgcn_readlane(a0, j), b1 = __builtin_amdgcn_readlane(a1, j);
-    any = any || (j != l && lv.ok && __builtin_amdgcn_readlane(lv.ok, j) && a0 < b1 && b0 < a1);
-  }
+  const bool any = wave_levels_overlap(p.L, l, lv);
   const int inc = wave_inclusive_scan(nt);
   t.base = inc - nt;
   const int ntiles = __builtin_amdgcn_readlane(inc, kWave - 1);

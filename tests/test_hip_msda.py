@@ -447,6 +447,28 @@ def test_overlapping_levels_sum_into_grad_value(device, levels, starts, S, dtype
                                  softmax=softmax, dtype=dtype, label=f"overlap {levels} {starts} {path}")
 
 
+@pytest.mark.parametrize("dtype", [F32, F64], ids=["f32", "f64"])
+@pytest.mark.parametrize(("count", "overlap"), [
+    (1, 0), (2, 0), (2, 3), (63, 0), (64, 0), (64, 3), (65, 0), (65, 3), (130, 0),
+])
+def test_level_tables_of_every_length(device, count, overlap, dtype):
+    """The sort and the owners plan up to 64 levels in one wave, longer tables in a loop;
+    ``overlap`` positions of the last level belong to the one before it too."""
+    levels = [(3 + i % 5, 2 + i % 7) for i in range(count)]
+    starts = [sum(h * w for h, w in levels[:i]) for i in range(count)]
+    starts[-1] -= overlap
+    g = torch.Generator().manual_seed(23)
+    B, Q, H, D, P = 1, 40, 2, 16, 3
+    value = torch.randn(B, starts[-1] + levels[-1][0] * levels[-1][1], H, D, generator=g, dtype=F64)
+    loc = torch.rand(B, Q, H, count, P, 2, generator=g, dtype=F64) * 1.1 - 0.05
+    attn = torch.softmax(torch.randn(B, Q, H, count * P, generator=g, dtype=F64), -1)
+    grad_out = torch.randn(B, Q, H * D, generator=g, dtype=F64)
+    ops = [t.to(device, dtype) for t in (value, loc, attn, grad_out)]
+    for softmax in (False, True):
+        check_against_oracle(ops[0], torch.tensor(levels, device=device), torch.tensor(starts, device=device), ops[1],
+                             ops[2], ops[3], softmax=softmax, dtype=dtype, label=f"{count} levels")
+
+
 def abi_backward_into(lib, w, grads, flags, stream, workspace=None):
     """One msda_backward call (workspace None) or msda_backward_workspace call on the
     workload's operands, writing into ``grads`` = (grad_value, grad_loc, grad_attn)."""
