@@ -2362,10 +2362,10 @@ __global__ __launch_bounds__(kOwnerThreads) void msda_grad_value_kernel(
         if constexpr (SOFTMAX) {
           const uint32_t q = fdiv(c_own, bg.div_lp), s = c_own - q * uint32_t(LP);
           const int64_t u = unit0 + int64_t(q) * p.H;
+          const A logit = load_acc(attn_all + u * LP + s);  // beside the statistics, whatever they say
           SoftStat<A> st{A(NAN)};
           if (stats) st = stats[u];
-          a = st.ok() ? exp_acc(load_acc(attn_all + u * LP + s) - st.lse)
-                      : unit_weight<T, true>(attn_all + u * LP, LP, int(s));
+          a = st.ok() ? exp_acc(logit - st.lse) : unit_weight<T, true>(attn_all + u * LP, LP, int(s));
         } else {
           a = to_acc(c_attn);
         }
