@@ -3931,6 +3931,11 @@ const char* dtype_name(int dtype) {
 // B = 2, Q = 5,376, 93 against 120 for 40 samples; float's 3 KB for 12 stay whole, 238
 // against 257 us in chunks of 8).
 constexpr int64_t kChunkBytesForward = 8192;
+// The forward stages whole while the LDS of its whole grid is this small: the chunks are
+// there for more waves per CU, and a grid that fits the chip's 40 MB has no more to bring.
+// Chunks against whole: 7.5 / 7.2 us at 5 MB, 15.2 / 14.6 at 12, 20.9 / 20.4 at 25, but 14.7
+// / 15.9 at 31 and 17.6 / 25.5 at 41 (16-bit values, 300 to 5,376 queries).
+constexpr int64_t kChunkGridBytes = int64_t(24) << 20;
 constexpr int64_t kChunkBytesBackward = 4096;
 
 struct Plan {
@@ -3983,12 +3988,6 @@ int make_plan(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t Q, 
   // and weights. When one wave's units do not fit, a unit takes more lanes (the
   // lanes past the channels stage samples and idle in the gathers), so a wave holds
   // fewer units.
-  auto chunk_for = [&](int lhl) {
-    const int64_t lh = int64_t(1) << lhl, bytes = (int64_t(kWave) >> lhl) * L * P * int64_t(staged);
-    const int64_t most = backward ? kChunkBytesBackward : kChunkBytesForward;
-    const int64_t n = (bytes + most - 1) / most;
-    return n <= 1 ? L * P : std::min<int64_t>(L * P, ((L * P + n - 1) / n + lh - 1) / lh * lh);
-  };
   auto lds_for = [&](int lhl, int w, int64_t chunk) {
     const int u = kWave >> lhl;
     const size_t per_wave = size_t(u) * size_t(chunk) * staged;
@@ -4004,8 +4003,15 @@ int make_plan(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t Q, 
                 "wave (%zu bytes needed)",
                 (long long)(L * P), kMaxLds, whole());
   const int uw = kWave >> lh_log2;
-  auto lds_of = [&](int w) { return lds_for(lh_log2, w, chunk_for(lh_log2)); };
   const int64_t units = Q * H;
+  const int64_t chunk = [&] {
+    const int64_t lh = int64_t(1) << lh_log2, bytes = int64_t(uw) * L * P * int64_t(staged);
+    if (!backward && B * ((units + uw - 1) / uw) <= kChunkGridBytes / int64_t(whole())) return L * P;
+    const int64_t most = backward ? kChunkBytesBackward : kChunkBytesForward;
+    const int64_t n = (bytes + most - 1) / most;
+    return n <= 1 ? L * P : std::min<int64_t>(L * P, ((L * P + n - 1) / n + lh - 1) / lh * lh);
+  }();
+  auto lds_of = [&](int w) { return lds_for(lh_log2, w, chunk); };
   int waves = kMaxWavesPerBlock;
   // Fewer waves per workgroup when the grid would leave CUs idle or LDS is short.
   while (waves > 1) {
@@ -4015,7 +4021,7 @@ int make_plan(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t Q, 
   }
   plan->cv = cv;
   plan->lh_log2 = lh_log2;
-  plan->chunk = int(chunk_for(lh_log2));
+  plan->chunk = int(chunk);
   plan->waves = waves;
   plan->units_per_block = waves * uw;
   plan->blocks_per_batch = int((units + plan->units_per_block - 1) / plan->units_per_block);

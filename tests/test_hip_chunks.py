@@ -1,8 +1,8 @@
-"""Samples staged in chunks (the forward beyond 8 KB of records a wave, grad_sample beyond
-4 KB), at the sizes where it can go wrong: a last chunk of one sample, chunks that end
-inside a level, samples that are no multiple of a unit's lanes, one or several chunks
-(with and without the barrier that keeps a workgroup's waves in step), every dtype. And
-grad_sample's 8-byte location gradient stores against its 4-byte ones.
+"""Samples staged in chunks (the forward beyond 8 KB of records a wave and 24 MB a grid,
+grad_sample beyond 4 KB), at the sizes where it can go wrong: a last chunk of one sample,
+chunks that end inside a level, samples that are no multiple of a unit's lanes, one or
+several chunks (with and without the barrier that keeps a workgroup's waves in step),
+every dtype. And grad_sample's 8-byte location gradient stores against its 4-byte ones.
 
 Tolerances are the parity suite's (float32 1e-5 forward, 1e-4 backward; 16-bit 2e-2 of the
 largest element; float64 1e-10); the stores must agree bit for bit.
@@ -14,6 +14,7 @@ import pytest
 import torch
 
 from deformops_amd.backends.hip import _lib
+from deformops_amd.registry import msda
 from tests.test_hip_msda import check_against_oracle
 from tests.workloads import make_workload
 
@@ -35,6 +36,33 @@ def test_chunked_staging_matches_the_oracle(device, levels, points, channels, dt
                       locations="uniform", seed=3).to(device, dtype, loc_dtype)
     check_against_oracle(*w.operands(softmax=softmax), w.grad_output, softmax=softmax, dtype=dtype,
                          label=f"L={levels} P={points} D={channels}")
+
+
+@pytest.mark.parametrize("softmax", [False, True], ids=["linear", "softmax"])
+@pytest.mark.parametrize(("dtype", "loc_dtype"), [(F32, F32), (BF16, F32), (F16, F16), (F64, F64)],
+                         ids=["f32", "bf16-f32loc", "f16", "f64"])
+@pytest.mark.parametrize(("levels", "points", "channels"), [
+    (1, 33, 32), (3, 7, 16), (5, 8, 32), (5, 5, 64), (2, 33, 16), (5, 13, 8), (4, 16, 128), (5, 4, 24),
+])
+def test_forward_in_chunks_equals_the_forward_staged_whole(device, levels, points, channels, dtype, loc_dtype, softmax):
+    """A grid of up to 24 MB of records is staged whole, a larger one in chunks: the same call
+    repeated over the batch gives the same bits."""
+    w = make_workload(2, batch=2, queries=203, heads=3, channels=channels, points=points, levels=LEVELS[:levels],
+                      locations="uniform", seed=6).to(device, dtype, loc_dtype)
+    value, shapes, starts, loc, attn = w.operands(softmax=softmax)
+    samples = levels * points
+    per_call = 2 * 203 * 3 * samples * (dtype.itemsize + 2 * loc_dtype.itemsize + (48 if dtype is F64 else 32))
+    whole, many = (24 << 20) // per_call // 2, (24 << 20) // per_call + 2
+    assert whole >= 1
+
+    def forward(times):
+        v, x, a = (t.repeat(times, *[1] * (t.dim() - 1)) for t in (value, loc, attn))
+        return msda(v, shapes, starts, x, a, softmax=softmax)
+
+    want = forward(1)
+    for times in (whole, many):
+        got = forward(times).view(times, *want.shape)
+        torch.testing.assert_close(got, want.expand_as(got), rtol=0, atol=0)
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16-f32loc"])
