@@ -1039,11 +1039,22 @@ __device__ inline bool wave_levels_overlap(int L, int l, const Level& lv) {
 // with atomics.
 __device__ inline int64_t load_tiles(const Problem& p, const BwdGeom& bg, Level* levels,
                                      LevelTiles* lt, int64_t* total_out, bool* overlap = nullptr) {
-  // By the first wave, a lane for each of 64 levels, in registers, with one barrier: the
-  // backward of B = 4, 300 queries, D = 24, four levels of three points takes 62 us, 65 with
-  // the tiles numbered by one thread behind two barriers more.
+  // One barrier. A single level by one thread, whose loads and arithmetic the compiler makes
+  // scalar: backward of B = 4, 4,096 queries, H = 3, D = 24, three points in float 53.9 us,
+  // 57.7 by the wave below. Otherwise by the first wave, a lane for each of 64 levels, in
+  // registers: 63.6 us for B = 4, 300 queries, D = 8 and four levels, 80.7 by one thread.
   const int lane = int(threadIdx.x);
-  if (lane < kWave) {
+  if (p.L == 1) {
+    if (lane == 0) {
+      const Level lv = load_level(p, 0);
+      const LevelTiles t = level_tiles(p, bg, lv);
+      const int64_t total = int64_t(t.ntx) * t.nty;
+      levels[0] = lv;
+      lt[0] = t;
+      *overlap_flag() = 0;
+      *total_out = total <= (int64_t(1) << 29) ? total : -1;
+    }
+  } else if (lane < kWave) {
     int64_t total = 0;
     bool any = false;
     for (int l0 = 0; l0 < p.L; l0 += kWave) {
